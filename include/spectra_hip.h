@@ -229,6 +229,16 @@ int spectra_quantize_nf4(const void* w, int64_t ldw, int32_t w_dtype, int64_t n,
                          uint8_t* packed, uint16_t* absmax, spectra_stream_t stream);
 
 /*
+ * CSR positions of a boolean mask [n, k] (bytes 0 or 1, row stride ldm): rowptr int32 [n + 1], and,
+ * once rowptr is known, col int32 [rowptr[n]] (ascending per row).  No reference code (Format B's
+ * side tensor).  The total must be below 2^31.
+ */
+int spectra_mask_rowptr(const uint8_t* mask, int64_t ldm, int64_t n, int64_t k, int32_t* rowptr,
+                        spectra_stream_t stream);
+int spectra_mask_columns(const uint8_t* mask, int64_t ldm, int64_t n, int64_t k, const int32_t* rowptr, int32_t* col,
+                         spectra_stream_t stream);
+
+/*
  * Blockwise normalised FWHT of rows (compressor.py:29-42), fp32 arithmetic in the
  * reference's butterfly order, division by fp32(sqrt(block)).
  * x [rows, k] in_dtype (row stride ldx) -> out [rows, k] out_dtype (row stride ldo).

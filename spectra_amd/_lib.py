@@ -69,6 +69,8 @@ SIGNATURES = {
                                            c_int32, c_void_p, c_void_p, c_void_p, c_void_p]),
     "spectra_quantize_nf4": (c_int32, [c_void_p, c_int64, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32,
                                        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "spectra_mask_rowptr": (c_int32, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p]),
+    "spectra_mask_columns": (c_int32, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p]),
     "spectra_fwht_rows": (c_int32, [c_void_p, c_int64, c_int32, c_int64, c_int64, c_int32, c_void_p, c_int64,
                                     c_int32, c_void_p]),
     "spectra_w4_embedding": (c_int32, [ctypes.POINTER(QWeight), c_void_p, c_int64, c_void_p, c_int64, c_int32,

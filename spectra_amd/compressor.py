@@ -145,6 +145,19 @@ class NF4Weight:
 def csr_from_mask(mask: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """Row-major CSR positions (rowptr int32 [N+1], col int32 [nnz]) of a boolean mask, on its device."""
     n = mask.shape[0]
+    if mask.is_cuda and mask.dtype == torch.bool and mask.dim() == 2 and mask.numel() > 0:
+        m = mask if mask.stride(1) == 1 and mask.stride(0) >= mask.shape[1] else mask.contiguous()
+        k, lib = m.shape[1], L.load()
+        with torch.cuda.device(m.device):
+            rowptr = torch.empty(n + 1, dtype=torch.int32, device=m.device)
+            L.check("spectra_mask_rowptr", lib.spectra_mask_rowptr(m.data_ptr(), m.stride(0) if n > 1 else k, n, k,
+                                                                   rowptr.data_ptr(), _stream(m.device)))
+            col = torch.empty(int(rowptr[-1]), dtype=torch.int32, device=m.device)  # the one host read
+            if col.numel():
+                L.check("spectra_mask_columns", lib.spectra_mask_columns(
+                    m.data_ptr(), m.stride(0) if n > 1 else k, n, k, rowptr.data_ptr(), col.data_ptr(),
+                    _stream(m.device)))
+        return rowptr, col
     rows, cols = torch.nonzero(mask, as_tuple=True)
     counts = torch.bincount(rows, minlength=n)
     rowptr = torch.zeros(n + 1, dtype=torch.int64, device=mask.device)
