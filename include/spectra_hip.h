@@ -309,6 +309,17 @@ int spectra_attend_decode(const void* qkv, const int64_t* pos, const float* cos_
                           int32_t kv_heads, int32_t head_dim, int32_t max_seq, void* k_cache, void* v_cache,
                           void* workspace, size_t workspace_bytes, void* out, spectra_stream_t stream);
 
+/* Causal attention of a prompt: out[t, h, :] = softmax(q[t, h] k^T / sqrt(head_dim)) v over
+ * positions [0, pos[t]] (fp32 scores and softmax; pos device int64 [tokens]) for the rotated
+ * queries q [tokens, heads, head_dim] (spectra_rope_append) and the caches [kv_heads, max_seq,
+ * head_dim], of which positions 0 .. keys - 1 are read (a query's later ones masked); out
+ * [tokens, heads, head_dim].  fp16, 16-byte aligned; head_dim 64 or 128
+ * (SPECTRA_ERR_UNSUPPORTED otherwise).  In the reference the prompt's attention is the model's
+ * own (engine.py:1387-1415 keeps its static cache). */
+int spectra_attend_prefill(const void* q, const int64_t* pos, int64_t tokens, int64_t keys, int32_t heads,
+                           int32_t kv_heads, int32_t head_dim, int32_t max_seq, const void* k_cache,
+                           const void* v_cache, void* out, spectra_stream_t stream);
+
 /* The 4-bit KV cache (engine.py:614-680 SpectraGroup32QuantizedLayer / :683-700
  * SpectraQuantizedCache).  Quantizer: per row of the head dimension, groups of 32,
  * asymmetric min-max codes 0..15 with fp16 scale and uint8 zero point, two codes per byte

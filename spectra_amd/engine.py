@@ -18,6 +18,7 @@ import torch.nn as nn
 
 from . import _lib as L
 from .kernels import (GEMV_MAX_M, QWeightOperands, argmax_slots, attend_decode, attend_decode_q4,
+                      attend_prefill,
                       attend_workspace_bytes, greedy_finish, greedy_next, kv4_quantize, rmsnorm, rope_append, silu_mul,
                       w4_embedding, w4a16_gemv_fused, w4a16_linear)
 
@@ -268,7 +269,8 @@ class SpectraDecoder(nn.Module):
     lm_head (engine.py:1124-1168) and an fp16 KV cache.  Between the linears a layer runs
     the library's fused kernels (residual add + RMSNorm, RoPE + cache append, split-sequence
     decode attention, SiLU-mul) where the reference relies on Inductor fusion
-    (engine.py:1240-1250); prefill attention over the prompt is a torch product.  A decode
+    (engine.py:1240-1250); so does the prompt (causal attention on the matrix cores for head
+    sizes 64 and 128, torch products for others).  A decode
     step is fully device-side (token, position and cache index live in device tensors), so
     it is captured once as a HIP graph and replayed per token (engine.py:1801-1860)."""
 
@@ -460,7 +462,6 @@ class SpectraDecoder(nn.Module):
         layer's output ``delta``; returns this layer's MLP output (added by the next norm)."""
         c, blk = self.cfg, self.blocks[li]
         hd, T = c.head_dim, h.shape[0]
-        g = c.heads // c.kv_heads
         x = rmsnorm(h, self.norm_w[2 * li], c.rms_eps, residual=delta)
         qkv = self._project(blk["qkv"], x)
         L = causal_len
@@ -480,6 +481,19 @@ class SpectraDecoder(nn.Module):
             last = self.arange[max(0, L - w):L]  # the window's positions -> ring slots position % window
             self.k_cache[li].index_copy_(1, last % w, kc[:, last])
             self.v_cache[li].index_copy_(1, last % w, vc[:, last])
+        if hd in (64, 128):
+            a = attend_prefill(q, pos, L, kc, vc).reshape(T, c.hidden)
+        else:
+            a = self._attend_products(q, kc, vc, pos, L)
+        o = blk["o"](a)
+        x = rmsnorm(h, self.norm_w[2 * li + 1], c.rms_eps, residual=o)
+        return blk["down"](silu_mul(self._project(blk["gate_up"], x)))
+
+    def _attend_products(self, q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, pos: torch.Tensor,
+                         L: int) -> torch.Tensor:
+        """Prefill attention as torch products, for the head sizes the kernel does not take."""
+        c = self.cfg
+        T, hd, g = q.shape[0], c.head_dim, c.heads // c.kv_heads
         qg = q.permute(1, 0, 2).reshape(c.kv_heads, g * T, hd).contiguous()  # head = kv * g + j
         kt = kc[:, :L, :].transpose(1, 2).contiguous()  # [kv, hd, L]
         vv = vc[:, :L, :].contiguous()
@@ -487,10 +501,7 @@ class SpectraDecoder(nn.Module):
         qpos = pos.repeat(g)  # row r = j * T + t -> position pos[t]
         s = s.masked_fill((self.arange[:L][None, :] > qpos[:, None])[None], float("-inf"))
         a = torch.matmul(torch.softmax(s, dim=-1).half(), vv)  # [kv, g*T, hd]
-        a = a.reshape(c.heads, T, hd).permute(1, 0, 2).reshape(T, c.hidden)
-        o = blk["o"](a)
-        x = rmsnorm(h, self.norm_w[2 * li + 1], c.rms_eps, residual=o)
-        return blk["down"](silu_mul(self._project(blk["gate_up"], x)))
+        return a.reshape(c.heads, T, hd).permute(1, 0, 2).reshape(T, c.hidden)
 
     @staticmethod
     def _project(parts, x: torch.Tensor) -> torch.Tensor:

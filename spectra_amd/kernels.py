@@ -28,7 +28,7 @@ from . import _lib as L
 
 __all__ = ["fused_w4a16_gemv_hdsq", "batched_w4a16_gemm", "w4a16_linear", "w4_dequant", "fwht_rows",
            "QWeightOperands", "GEMV_MAX_M", "w4_embedding", "rmsnorm", "rope_append", "attend_decode",
-           "attend_workspace_bytes", "silu_mul", "greedy_next", "argmax_slots", "greedy_finish",
+           "attend_workspace_bytes", "attend_prefill", "silu_mul", "greedy_next", "argmax_slots", "greedy_finish",
            "w4a16_gemv_fused", "kv4_quantize",
            "kv4_dequantize", "attend_decode_q4", "validate_outliers"]
 
@@ -508,6 +508,32 @@ def attend_decode(qkv: torch.Tensor, pos: torch.Tensor, cos: Optional[torch.Tens
         qkv.data_ptr(), pos.data_ptr(), cos.data_ptr() if cos is not None else None,
         sin.data_ptr() if sin is not None else None, heads, kv, hd, lmax, k_cache.data_ptr(), v_cache.data_ptr(),
         workspace.data_ptr(), workspace.numel() * workspace.element_size(), out.data_ptr(), _stream(qkv.device)))
+    return out
+
+
+def attend_prefill(q: torch.Tensor, pos: torch.Tensor, keys: int, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Causal attention of T prompt tokens at positions ``pos`` (int64 [T] on the device): rotated
+    queries ``q`` [T, heads, d] over the first ``keys`` rows of the caches [kv, L, d] (fp16, d 64
+    or 128), each query over [0, its position]; returns fp16 [T, heads, d]."""
+    _need_f16(q, "q")
+    _need_f16(k_cache, "k_cache")
+    _need_f16(v_cache, "v_cache")
+    kv, lmax, hd = k_cache.shape
+    T, heads, d = q.shape
+    if pos.dtype != torch.int64 or not pos.is_cuda or not pos.is_contiguous() or pos.numel() != T:
+        raise ValueError("pos must be contiguous int64 [T] on the GPU")
+    if v_cache.shape != k_cache.shape or d != hd or heads % kv:
+        raise ValueError("q must be [T, heads, d] and the caches [kv_heads, L, d]")
+    if out is None:
+        out = torch.empty_like(q)
+    _need_f16(out, "out")
+    if out.shape != q.shape:
+        raise ValueError("out must have q's shape")
+    lib = L.load()
+    L.check("spectra_attend_prefill", lib.spectra_attend_prefill(q.data_ptr(), pos.data_ptr(), T, int(keys), heads, kv, hd, lmax,
+                                                                 k_cache.data_ptr(), v_cache.data_ptr(),
+                                                                 out.data_ptr(), _stream(q.device)))
     return out
 
 
