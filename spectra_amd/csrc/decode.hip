@@ -19,6 +19,7 @@
 //
 // The position of the decoded token is read from device memory, so a decode step has no
 // host-side value and is captured once as a HIP graph.
+#include <algorithm>
 #include <cmath>
 
 #include "common.h"
@@ -279,10 +280,11 @@ __device__ __forceinline__ float load_dev(const float* p) {
 // exponentials and turns the batch into weights exp(m - M) (m = -inf marks an empty span,
 // weight 0) in LDS; every thread loads the V sums of its outputs (o, o + 256, ...) and folds
 // them in with those weights.
-template <int HD>
+template <int HD, int NT = kDecThreads, int B = 16>
 __device__ __forceinline__ void attend_arrive_merge(const float* part, uint32_t* counter, uint16_t* out, int kh,
                                                     int G, int nspan, int tid, int* last_l) {
-  constexpr int B = 16, GM = 8, O = (GM * HD + kDecThreads - 1) / kDecThreads;
+  constexpr int GM = 8, O = (GM * HD + NT - 1) / NT;
+  static_assert((B == 16 || B == 32) && NT >= GM * B, "one weight lane per head and piece of a batch");
   __shared__ __align__(16) float fw[GM][B + 4];  // the batch's span weights per head, then the rescale
   __shared__ float hl_s[GM];
   __builtin_amdgcn_s_waitcnt(0);
@@ -312,7 +314,7 @@ __device__ __forceinline__ void attend_arrive_merge(const float* part, uint32_t*
     float av[O][B];
 #pragma unroll
     for (int q = 0; q < O; ++q) {
-      const int o = tid + q * kDecThreads;
+      const int o = tid + q * NT;
       const int oc = o < total ? o : 0;
       const int j = oc / HD, d = oc - j * HD;
       const float* pj = ph0 + (int64_t)j * nspan * (HD + 2) + d;
@@ -325,6 +327,7 @@ __device__ __forceinline__ void attend_arrive_merge(const float* part, uint32_t*
       mb = fmaxf(mb, lane_xor<2>(mb, lane));
       mb = fmaxf(mb, lane_xor<4>(mb, lane));
       mb = fmaxf(mb, lane_xor<8>(mb, lane));
+      if constexpr (B > 16) mb = fmaxf(mb, lane_xor<16>(mb, lane));
       mb = fmaxf(mb, hm);
       const float r = mb == -INFINITY ? 1.0f : __expf(hm - mb);  // rescale of what came before (0 if nothing)
       const float f = wmv == -INFINITY ? 0.0f : __expf(wmv - mb);  // empty span: weight 0
@@ -333,6 +336,7 @@ __device__ __forceinline__ void attend_arrive_merge(const float* part, uint32_t*
       lb += lane_xor<2>(lb, lane);
       lb += lane_xor<4>(lb, lane);
       lb += lane_xor<8>(lb, lane);
+      if constexpr (B > 16) lb += lane_xor<16>(lb, lane);
       hl = hl * r + lb;
       hm = mb;
       fw[wj][wu] = f;
@@ -341,7 +345,7 @@ __device__ __forceinline__ void attend_arrive_merge(const float* part, uint32_t*
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < O; ++q) {
-      const int o = tid + q * kDecThreads;
+      const int o = tid + q * NT;
       if (o < total) {
         const int j = o / HD;
         float t = a[q] * fw[j][B];
@@ -359,7 +363,7 @@ __device__ __forceinline__ void attend_arrive_merge(const float* part, uint32_t*
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < O; ++q) {
-    const int o = tid + q * kDecThreads;
+    const int o = tid + q * NT;
     if (o < total) out[(int64_t)kh * G * HD + o] = f2h(a[q] / hl_s[o / HD]);
   }
 }
@@ -590,8 +594,9 @@ __global__ void __launch_bounds__(kDecThreads) attend_kernel(const uint16_t* __r
 }
 
 // MFMA decode attention on the fp16 cache (head_dim 64, 128 or 256, at most 8 query heads
-// per KV head).  Same grid, spans, partials and merge as attend_kernel; inside a span
-// workgroup wave w takes positions t0 + 16 w .. + 15 and lane (i, g) = (lane & 15, lane >> 4):
+// per KV head).  Same spans, partials and merge as attend_kernel; workgroup sp of the grid
+// of NW waves takes the spans sp, sp + gridDim.y, ... of 16 NW positions up to the position, and
+// inside a span wave w takes positions t0 + 16 w .. + 15 and lane (i, g) = (lane & 15, lane >> 4):
 //   * holds the 16-byte chunks 32 c + 8 g .. + 7 (c < head_dim / 32) of position t0 + 16 w + i
 //     for K and V, and of query head i for q (zero for i >= G): the A and B operands of
 //     v_mfma_f32_16x16x32_f16, so scores = K q^T is head_dim / 32 MFMAs;
@@ -607,10 +612,11 @@ __global__ void __launch_bounds__(kDecThreads) attend_kernel(const uint16_t* __r
 typedef _Float16 ah8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 ah4_t __attribute__((ext_vector_type(4)));
 typedef float af4_t __attribute__((ext_vector_type(4)));
+constexpr int kAttendGrid = 32;   // most workgroups per KV head of attend_mfma_kernel
 constexpr int kMfmaMaxGroup = 8;  // query heads per KV head served by attend_mfma_kernel
 
-template <int HD, bool ROPE>
-__global__ void __launch_bounds__(kDecThreads) attend_mfma_kernel(const uint16_t* __restrict__ qkv,
+template <int HD, bool ROPE, int NW>
+__global__ void __launch_bounds__(64 * NW) attend_mfma_kernel(const uint16_t* __restrict__ qkv,
                                                                    const int64_t* __restrict__ pos_p,
                                                                    const float* __restrict__ cos_t,
                                                                    const float* __restrict__ sin_t, int heads,
@@ -623,13 +629,16 @@ __global__ void __launch_bounds__(kDecThreads) attend_mfma_kernel(const uint16_t
   constexpr int VS = HD + 8;   // LDS row stride (halves) of the V tiles and the rotated rows
   constexpr int GM = kMfmaMaxGroup;
   constexpr int RB = HD / 16;  // rotation work items per row (8 pairs (d, d + HD / 2) each)
+  constexpr int SP = 16 * NW;  // positions of a span
+  constexpr int MB = NW == 4 ? 16 : 32;  // pieces the merge takes at once
+  constexpr bool LOOP = NW > 4;  // (grids of 4-wave workgroups have one span each)
   static_assert(HD == 64 || HD == 128 || HD == 256, "head_dim 64, 128 or 256");
   // the V tiles [wave][16][VS] (fp16), then, once every wave is past its P V, the per-wave
   // V sums [wave][GM][HD] (fp32) in the same bytes
-  __shared__ __align__(16) uint8_t lds[4 * 16 * VS * 2];
-  static_assert(4 * GM * HD * 4 <= 4 * 16 * VS * 2, "per-wave V sums fit the V tiles");
+  __shared__ __align__(16) uint8_t lds[NW * 16 * VS * 2];
+  static_assert(GM * HD * 4 <= 16 * VS * 2, "per-wave V sums fit the V tiles");
   __shared__ __align__(16) uint16_t qs[GM + 1][VS];  // rotated query heads, then the new key
-  __shared__ float wm[4][16], wl[4][16];              // per-wave max and sum of exponentials
+  __shared__ float wm[NW][16], wl[NW][16];              // per-wave max and sum of exponentials
   __shared__ int last_l;
   // every kernel argument in one round trip, before the first load
   asm volatile("" ::"s"(qkv), "s"(pos_p), "s"(cos_t), "s"(sin_t), "s"(heads), "s"(kv_heads), "s"(scale),
@@ -638,13 +647,12 @@ __global__ void __launch_bounds__(kDecThreads) attend_mfma_kernel(const uint16_t
   const int lmax = kvc.lmax;
   const int kh = blockIdx.x, sp = blockIdx.y, nspan = gridDim.y, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, i16 = lane & 15, g4 = lane >> 4;
-  const int t0 = sp * kSpanMax;
-  const int tp = t0 + 16 * wave + i16;  // the position of this lane's K / V chunks
+  const int wp = 16 * wave + i16;  // this lane's row of a span
   // rotation item of this lane: row i (< G: query head, G: the new key), pair block
   // b = RBW w + g (pairs (d, d + HD / 2), d = 8 b .. + 7); its query / key halves load first,
   // so that waiting for them waits for no K / V chunk
-  constexpr int RBW = RB / 4;  // pair blocks per wave
-  const bool ritem = g4 < RBW && i16 <= G;
+  constexpr int RBW = RB / 4;  // pair blocks per wave (of the first four)
+  const bool ritem = wave < 4 && g4 < RBW && i16 <= G;
   const int rblk = RBW * wave + g4;
   uint4 rlo = make_uint4(0, 0, 0, 0), rhi = rlo;
   if (ritem) {
@@ -656,34 +664,35 @@ __global__ void __launch_bounds__(kDecThreads) attend_mfma_kernel(const uint16_t
   const uint16_t* kbase = kvc.k + (int64_t)kh * lmax * HD;
   const uint16_t* vbase = kvc.v + (int64_t)kh * lmax * HD;
   uint4 kr[KI], vr[KI];
-  {
-    const uint32_t o = (uint32_t)(min(tp, lmax - 1) * HD + 8 * g4) * 2u;
+  auto load_span = [&](int t0, uint4 (&k)[KI], uint4 (&v)[KI]) __attribute__((always_inline)) {
+    const uint32_t o = (uint32_t)(min(t0 + wp, lmax - 1) * HD + 8 * g4) * 2u;
 #pragma unroll
     for (int c = 0; c < KI; ++c) {
-      kr[c] = load_at<uint4>(kbase, o + 64u * c);
-      vr[c] = load_at<uint4>(vbase, o + 64u * c);
+      k[c] = load_at<uint4>(kbase, o + 64u * c);
+      v[c] = load_at<uint4>(vbase, o + 64u * c);
     }
-  }
+  };
+  load_span(sp * SP, kr, vr);
   asm volatile("" ::: "memory");  // the K / V chunks are requested here, not sunk behind the position
   // the position: a scalar load (it waits for no vector load)
   const int64_t pos = *(const __attribute__((address_space(4))) int64_t*)pos_p;
   const bool outside = pos < 0 || pos >= lmax;
-  const int n = outside ? 0 : (int)min((int64_t)kSpanMax, pos + 1 - t0);  // uniform
+  const int last = outside ? -1 : (int)pos;  // uniform
   float* pbase = part + ((int64_t)kh * G * nspan + sp) * (HD + 2);     // head j: + j * nspan * (HD + 2)
-  if (n <= 0) {  // span past the position: an empty piece for the merge
+  if (sp * SP > last) {  // its first span past the position: an empty piece for the merge
     if (tid < G) {
       store_dev(pbase + (int64_t)tid * nspan * (HD + 2) + HD, -INFINITY);
       store_dev(pbase + (int64_t)tid * nspan * (HD + 2) + HD + 1, 0.0f);
     }
-    attend_arrive_merge<HD>(part, counter, out, kh, G, nspan, tid, &last_l);
+    attend_arrive_merge<HD, 64 * NW, MB>(part, counter, out, kh, G, nspan, tid, &last_l);
     return;
   }
   // ---- rotation: the cos / sin of the position for the wave's pair blocks (scalar loads:
   //      they wait for no vector load), the rope_append arithmetic, into LDS
   if constexpr (ROPE) {
     typedef const __attribute__((address_space(4))) float* cfp_t;
-    const cfp_t ct = (cfp_t)(cos_t + pos * (HD / 2) + 8 * RBW * wave);
-    const cfp_t st = (cfp_t)(sin_t + pos * (HD / 2) + 8 * RBW * wave);
+    const cfp_t ct = (cfp_t)(cos_t + pos * (HD / 2) + 8 * RBW * (wave & 3));
+    const cfp_t st = (cfp_t)(sin_t + pos * (HD / 2) + 8 * RBW * (wave & 3));
     float cw[8 * RBW], sw[8 * RBW];
 #pragma unroll
     for (int e = 0; e < 8 * RBW; ++e) {
@@ -712,7 +721,8 @@ __global__ void __launch_bounds__(kDecThreads) attend_mfma_kernel(const uint16_t
     *(uint4*)&qs[i16][8 * rblk] = rlo;
     *(uint4*)&qs[i16][HD / 2 + 8 * rblk] = rhi;
   }
-  const bool mine = tp == pos;  // the lanes of the new token's row
+  // the new token's row: this lane's, when the span it lies in is one of this workgroup's
+  const bool mine = LOOP ? (last / SP) % nspan == sp && last % SP == wp : sp * SP + wp == last;
   uint4 vn[KI];
   if (mine) {
     const uint16_t* vrow = qkv + (int64_t)(heads + kv_heads + kh) * HD;
@@ -720,64 +730,96 @@ __global__ void __launch_bounds__(kDecThreads) attend_mfma_kernel(const uint16_t
     for (int c = 0; c < KI; ++c) vn[c] = load_at<uint4>(vrow, 16u * (4 * c + g4));
   }
   __syncthreads();
-  // ---- the new token: appended to the caches, and taken from registers
-  if (mine) {
-    const uint32_t o = (uint32_t)(pos * HD + 8 * g4) * 2u;
+  // ---- the spans sp, sp + nspan, ... up to the position; a span's V sums and softmax piece join
+  //      the wave's running ones (log-sum-exp) as the merge would join them
+  uint16_t* vt = (uint16_t*)lds + wave * 16 * VS;
+  float mx = -INFINITY, l = 0.0f;
+  af4_t acc[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b) acc[b] = af4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int t0 = sp * SP;;) {
+    const int n = min(SP, last + 1 - t0);
+    // ---- the new token: appended to the caches, and taken from registers
+    if (mine && t0 + wp == last) {
+      const uint32_t o = (uint32_t)(last * HD + 8 * g4) * 2u;
+#pragma unroll
+      for (int c = 0; c < KI; ++c) {
+        kr[c] = *(const uint4*)&qs[G][32 * c + 8 * g4];
+        vr[c] = vn[c];
+        *(uint4*)((uint8_t*)kvc.k + (int64_t)kh * lmax * HD * 2 + o + 64u * c) = kr[c];
+        *(uint4*)((uint8_t*)kvc.v + (int64_t)kh * lmax * HD * 2 + o + 64u * c) = vr[c];
+      }
+    }
+    // ---- this wave's V tile, rows past the position zeroed
+    {
+      const bool vok = wp < n;
+#pragma unroll
+      for (int c = 0; c < KI; ++c)
+        *(uint4*)(vt + i16 * VS + 32 * c + 8 * g4) = vok ? vr[c] : make_uint4(0, 0, 0, 0);
+    }
+    // ---- scores: D[position 4 g + r][head i]
+    af4_t sc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int c = 0; c < KI; ++c) {
-      kr[c] = *(const uint4*)&qs[G][32 * c + 8 * g4];
-      vr[c] = vn[c];
-      *(uint4*)((uint8_t*)kvc.k + (int64_t)kh * lmax * HD * 2 + o + 64u * c) = kr[c];
-      *(uint4*)((uint8_t*)kvc.v + (int64_t)kh * lmax * HD * 2 + o + 64u * c) = vr[c];
+      const uint4 qc = i16 < G ? *(const uint4*)&qs[i16][32 * c + 8 * g4] : make_uint4(0, 0, 0, 0);
+      sc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(ah8_t, kr[c]), __builtin_bit_cast(ah8_t, qc),
+                                                  sc, 0, 0, 0);
     }
-  }
-  // ---- this wave's V tile, rows past the position zeroed
-  uint16_t* vt = (uint16_t*)lds + wave * 16 * VS;
-  {
-    const bool vok = tp - t0 < n;
+    // ---- the wave's softmax piece for head i over its 16 positions
+    const int pb = 16 * wave + 4 * g4;  // span-relative position of row r = pb + r
+    float e[4];
+    float ms = -INFINITY;
 #pragma unroll
-    for (int c = 0; c < KI; ++c)
-      *(uint4*)(vt + i16 * VS + 32 * c + 8 * g4) = vok ? vr[c] : make_uint4(0, 0, 0, 0);
-  }
-  // ---- scores: D[position 4 g + r][head i]
-  af4_t sc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int r = 0; r < 4; ++r) {
+      e[r] = pb + r < n ? sc[r] * scale : -INFINITY;
+      ms = fmaxf(ms, e[r]);
+    }
+    ms = fmaxf(ms, lane_xor<16>(ms, lane));
+    ms = fmaxf(ms, lane_xor<32>(ms, lane));
+    float ls = 0.0f;
 #pragma unroll
-  for (int c = 0; c < KI; ++c) {
-    const uint4 qc = i16 < G ? *(const uint4*)&qs[i16][32 * c + 8 * g4] : make_uint4(0, 0, 0, 0);
-    sc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(ah8_t, kr[c]), __builtin_bit_cast(ah8_t, qc), sc,
-                                                0, 0, 0);
-  }
-  // ---- the wave's softmax piece for head i over its 16 positions
-  const int pb = 16 * wave + 4 * g4;  // span-relative position of row r = pb + r
-  float e[4];
-  float mx = -INFINITY;
+    for (int r = 0; r < 4; ++r) {
+      e[r] = pb + r < n ? __expf(e[r] - ms) : 0.0f;  // (no valid row: ms = -inf, every e 0)
+      ls += e[r];
+    }
+    ls += lane_xor<16>(ls, lane);
+    ls += lane_xor<32>(ls, lane);
+    // ---- P V: D[head 4 g + r][dim 16 b + i]
+    const ah4_t pa = {(_Float16)e[0], (_Float16)e[1], (_Float16)e[2], (_Float16)e[3]};
+    const uint16_t* vrd = vt + (4 * g4) * VS + i16;
+    float ro[4], rn[4];  // scales of head 4 g + r: what came before, this span
+    const bool first = !LOOP || t0 == sp * SP;
+    if (first) {
+      mx = ms;
+      l = ls;
+    } else {
+      const float mn = fmaxf(mx, ms);  // finite: a later span's workgroup has a whole first one
+      const float fo = __expf(mx - mn), fs = ms == -INFINITY ? 0.0f : __expf(ms - mn);
+      l = l * fo + ls * fs;
+      mx = mn;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    e[r] = pb + r < n ? sc[r] * scale : -INFINITY;
-    mx = fmaxf(mx, e[r]);
-  }
-  mx = fmaxf(mx, lane_xor<16>(mx, lane));
-  mx = fmaxf(mx, lane_xor<32>(mx, lane));
-  float l = 0.0f;
+      for (int r = 0; r < 4; ++r) {
+        ro[r] = __shfl(fo, 4 * g4 + r, 64);
+        rn[r] = __shfl(fs, 4 * g4 + r, 64);
+      }
+    }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    e[r] = pb + r < n ? __expf(e[r] - mx) : 0.0f;  // (no valid row: mx = -inf, every e 0)
-    l += e[r];
-  }
-  l += lane_xor<16>(l, lane);
-  l += lane_xor<32>(l, lane);
-  // ---- P V: D[head 4 g + r][dim 16 b + i]
-  const ah4_t pa = {(_Float16)e[0], (_Float16)e[1], (_Float16)e[2], (_Float16)e[3]};
-  af4_t acc[DB];
-  const uint16_t* vrd = vt + (4 * g4) * VS + i16;
+    for (int b = 0; b < DB; ++b) {
+      const ah4_t vb = {__builtin_bit_cast(_Float16, vrd[16 * b]), __builtin_bit_cast(_Float16, vrd[VS + 16 * b]),
+                        __builtin_bit_cast(_Float16, vrd[2 * VS + 16 * b]),
+                        __builtin_bit_cast(_Float16, vrd[3 * VS + 16 * b])};
+      const af4_t pv = __builtin_amdgcn_mfma_f32_16x16x16f16(pa, vb, af4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+      if (first)
+        acc[b] = pv;
+      else
 #pragma unroll
-  for (int b = 0; b < DB; ++b) {
-    const ah4_t vb = {__builtin_bit_cast(_Float16, vrd[16 * b]), __builtin_bit_cast(_Float16, vrd[VS + 16 * b]),
-                      __builtin_bit_cast(_Float16, vrd[2 * VS + 16 * b]),
-                      __builtin_bit_cast(_Float16, vrd[3 * VS + 16 * b])};
-    acc[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(pa, vb, af4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        for (int r = 0; r < 4; ++r) acc[b][r] = acc[b][r] * ro[r] + pv[r] * rn[r];
+    }
+    t0 += nspan * SP;
+    if (!LOOP || t0 > last) break;
+    load_span(t0, kr, vr);
   }
-  // ---- the four waves' pieces -> the span's partials: each wave's V sums (unscaled) and
+  // ---- the waves' pieces -> the span's partials: each wave's V sums (unscaled) and
   //      softmax piece to LDS, then per output the log-sum-exp combination in wave order
   if (g4 == 0) {
     wm[wave][i16] = mx;
@@ -794,24 +836,28 @@ __global__ void __launch_bounds__(kDecThreads) attend_mfma_kernel(const uint16_t
     }
   }
   __syncthreads();
-  for (int o = tid; o < G * HD; o += kDecThreads) {
+  for (int o = tid; o < G * HD; o += 64 * NW) {
     const int j = o / HD, d = o - j * HD;
-    const float m4 = fmaxf(fmaxf(wm[0][j], wm[1][j]), fmaxf(wm[2][j], wm[3][j]));
+    float m4 = wm[0][j];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m4 = fmaxf(m4, wm[w][j]);
     float a = 0.0f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) a += wm[w][j] == -INFINITY ? 0.0f : ws[(w * GM + j) * HD + d] * __expf(wm[w][j] - m4);
+    for (int w = 0; w < NW; ++w) a += wm[w][j] == -INFINITY ? 0.0f : ws[(w * GM + j) * HD + d] * __expf(wm[w][j] - m4);
     store_dev(pbase + (int64_t)j * nspan * (HD + 2) + d, a);
   }
   if (tid < G) {
     const int j = tid;
-    const float m4 = fmaxf(fmaxf(wm[0][j], wm[1][j]), fmaxf(wm[2][j], wm[3][j]));
+    float m4 = wm[0][j];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m4 = fmaxf(m4, wm[w][j]);
     float lt = 0.0f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) lt += wm[w][j] == -INFINITY ? 0.0f : wl[w][j] * __expf(wm[w][j] - m4);
+    for (int w = 0; w < NW; ++w) lt += wm[w][j] == -INFINITY ? 0.0f : wl[w][j] * __expf(wm[w][j] - m4);
     store_dev(pbase + (int64_t)j * nspan * (HD + 2) + HD, m4);
     store_dev(pbase + (int64_t)j * nspan * (HD + 2) + HD + 1, lt);
   }
-  attend_arrive_merge<HD>(part, counter, out, kh, G, nspan, tid, &last_l);
+  attend_arrive_merge<HD, 64 * NW, MB>(part, counter, out, kh, G, nspan, tid, &last_l);
 }
 
 // grid (ceil(rows * d / 8 / 256), heads): one lane per 8 values (groups of 32 = 4 lanes)
@@ -1064,6 +1110,14 @@ static attend_fn pick_attend_hd(int hd, int g) {
   }
 }
 
+template <int NW>
+static attend_fn pick_mfma(int hd, bool rope) {
+  if (rope) return hd == 64 ? attend_mfma_kernel<64, true, NW> : hd == 128 ? attend_mfma_kernel<128, true, NW>
+                                                                          : attend_mfma_kernel<256, true, NW>;
+  return hd == 64 ? attend_mfma_kernel<64, false, NW> : hd == 128 ? attend_mfma_kernel<128, false, NW>
+                                                                  : attend_mfma_kernel<256, false, NW>;
+}
+
 static int attend_launch(const void* qkv, const int64_t* pos, const float* cos_t, const float* sin_t, int32_t heads,
                          int32_t kv_heads, int32_t head_dim, const KvCache& kvc, bool q4, void* workspace,
                          size_t workspace_bytes, void* out, spectra_stream_t stream) {
@@ -1089,22 +1143,30 @@ static int attend_launch(const void* qkv, const int64_t* pos, const float* cos_t
     return fail(SPECTRA_ERR_WORKSPACE, "workspace missing, unaligned or smaller than spectra_attend_workspace()");
   const int g = heads / kv_heads;
   attend_fn fn;
+  const bool mfma = !q4 && g <= kMfmaMaxGroup && head_dim >= 64;
+  // One 64-position span a workgroup up to kAttendGrid of them; longer caches run 8 waves a
+  // workgroup on 128-position spans, then several spans each, so that the pieces a head's last
+  // workgroup merges stay at most kAttendGrid, one round trip.  128 dims, us a call, before and
+  // after: 24 / 8 heads, position 6001 of 8192, 20.9 and 13.0 (24.6 MB: 5.1 at the card's copy
+  // rate, on the 7.6 of a 700-position call); position 300 of 16384, 37.9 and 10.4; 32 / 4 heads,
+  // 15000 of 16384, 46.9 and 18.5.  16 waves took 14.1 / 14.6 / 18.3, 64 pieces 14.7 / 15.3 / 18.2,
+  // several spans on 4 waves 15.6 / 9.8 / 28.1; 1900 of 2048 takes 9.1 as it was.
+  int nspan = spectra_attend_spans(kvc.lmax);
+  const bool wide = mfma && nspan > kAttendGrid;
+  const int nw = wide ? 8 : 4;
+  if (wide) nspan = std::min((kvc.lmax + 16 * nw - 1) / (16 * nw), kAttendGrid);
   if (q4) fn = cos_t ? pick_attend_hd<true, true>(head_dim, g) : nullptr;
-  else if (g <= kMfmaMaxGroup && head_dim >= 64)  // the MFMA kernel
-    fn = cos_t ? (head_dim == 64 ? attend_mfma_kernel<64, true> : head_dim == 128 ? attend_mfma_kernel<128, true>
-                                                                                 : attend_mfma_kernel<256, true>)
-               : (head_dim == 64 ? attend_mfma_kernel<64, false> : head_dim == 128 ? attend_mfma_kernel<128, false>
-                                                                                  : attend_mfma_kernel<256, false>);
+  else if (mfma)
+    fn = wide ? pick_mfma<8>(head_dim, cos_t != nullptr) : pick_mfma<4>(head_dim, cos_t != nullptr);
   else fn = cos_t ? pick_attend_hd<true, false>(head_dim, g) : pick_attend_hd<false, false>(head_dim, g);
   if (fn == nullptr)
     return fail(SPECTRA_ERR_UNSUPPORTED, "decode attention serves 1, 2, 3, 4, 6 or 8 query heads per KV head "
                                          "(the 4-bit cache with RoPE)");
-  const int nspan = spectra_attend_spans(kvc.lmax);
   const float scale = 1.0f / sqrtf((float)head_dim);
   uint32_t* counter = (uint32_t*)workspace;
   float* part = (float*)((uint8_t*)workspace + attend_counter_bytes(heads));
   const hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(fn, dim3((unsigned)kv_heads, (unsigned)nspan), dim3(kDecThreads), 0, s, (const uint16_t*)qkv,
+  hipLaunchKernelGGL(fn, dim3((unsigned)kv_heads, (unsigned)nspan), dim3(64 * nw), 0, s, (const uint16_t*)qkv,
                      pos, cos_t, sin_t, heads, kv_heads, scale, kvc, part, counter, (uint16_t*)out);
   SPECTRA_HIP_CHECK(hipGetLastError());
   return SPECTRA_OK;
