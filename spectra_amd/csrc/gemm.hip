@@ -20,6 +20,7 @@
 //    each half-step interleaves the MFMAs of one step with the decode, tile writes and
 //    loads of the next (scheduling groups), so the matrix pipe is fed while the wave
 //    decodes.  The epilogue undoes the row scale, adds the bias in fp32 and rounds once.
+#include <algorithm>
 #include <cmath>
 
 #include "common.h"
@@ -724,6 +725,11 @@ size_t prefill_workspace(const spectra_qweight_t* w, int64_t m, int act_dtype);
 int prefill_launch(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m, int act_dtype, void* out,
                    int64_t ldo, void* workspace, size_t workspace_bytes, hipStream_t s);
 
+// mid.hip: mid-size batches (17 <= m < 512)
+size_t mid_workspace(const spectra_qweight_t* w, int64_t m, int64_t tile_wgs);
+int mid_launch(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m, int act_dtype, void* out,
+               int64_t ldo, void* workspace, size_t workspace_bytes, int64_t tile_wgs, hipStream_t s);
+
 // skinny.hip: the small-batch MFMA family (2 <= m <= 16)
 size_t skinny_workspace(const spectra_qweight_t* w, int64_t m);
 int skinny_launch(const spectra_qweight_t* w, const void* x, int64_t ldx, int64_t m, int act_dtype, void* out,
@@ -748,12 +754,19 @@ size_t gemm_workspace_min(const spectra_qweight_t* w, int64_t m) {
   const size_t small = skinny_workspace(w, m);
   return gemm > small ? gemm : small;
 }
+
+// workgroups gemm_kernel runs for m rows (mid.hip's dispatch rule)
+static int64_t tile_workgroups(const spectra_qweight_t* w, int64_t m) {
+  const GemmPlan g = plan_gemm(m, w->n, w->k);
+  return (int64_t)g.mt * g.nt * g.ksplit;
+}
 }  // namespace spectra
 
 extern "C" size_t spectra_w4a16_gemm_workspace(const spectra_qweight_t* w, int64_t m, int32_t act_dtype) {
   if (w == nullptr || m <= 0) return 0;
   const size_t need = gemm_workspace_min(w, m), lib = prefill_workspace(w, m, act_dtype);
-  return need > lib ? need : lib;
+  const size_t mid = mid_workspace(w, m, tile_workgroups(w, m));
+  return std::max(need, std::max(lib, mid));
 }
 
 extern "C" int spectra_w4a16_gemm(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m,
@@ -786,6 +799,9 @@ extern "C" int spectra_w4a16_gemm(const spectra_qweight_t* w, const void* a, int
     const int pst = prefill_launch(w, a, lda, m, act_dtype, out, ldo, workspace, workspace_bytes, s);
     if (pst != SPECTRA_ERR_UNSUPPORTED) return pst;
   }
+  // 17 .. 96 rows, to 160 without outliers, and shapes that leave this file's tiles few workgroups
+  const int mst = mid_launch(w, a, lda, m, act_dtype, out, ldo, workspace, workspace_bytes, tile_workgroups(w, m), s);
+  if (mst != SPECTRA_ERR_UNSUPPORTED) return mst;
   uint16_t* a16 = (uint16_t*)workspace;
   int32_t* fexp = (int32_t*)((uint8_t*)workspace + align256((size_t)m * w->k * 2));
   const int had = w->hadamard_block;

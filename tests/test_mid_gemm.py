@@ -1,0 +1,120 @@
+"""The mid-size batch family (17 rows up to 96, 160 without outliers, 511 on shapes with few tiles)
+against the float64 product of W_eff, at the edges of its tiles: 32-row tiles and the change from
+four chunks a stage to two and to one, columns past the last 128, K of an odd number of 64-chunks and
+of a partial quad, every number of K splits' remainder, both formats and nibble orders, rotation
+blocks, dense and empty outlier rows, codes under the outliers that are not zero, unaligned and
+strided operands.  Bound: fp16 operands (weights and activations rounded once, 2^-11 each) and the
+result's rounding: rel-L2 <= 1e-3 in fp16, 5e-3 in bf16, as for the GEMM family."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from spectra_amd import _lib as L
+from spectra_amd import compressor as C
+from spectra_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+DT = {"float16": torch.float16, "bfloat16": torch.bfloat16}
+
+
+def _nf4(n, k, had, ratio, marlin, bs=64, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed + n + k)
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    mask = None
+    if ratio:
+        mask = torch.rand(n, k, generator=g, device="cuda") < ratio
+        mask[0] = False
+        mask[n - 1, : k // 2] = True
+        w = torch.where(mask, w * 10, w)
+    return C.quantize_nf4(w.half(), bs, 0, mask, marlin), had
+
+
+def _dense(q, bs=64):
+    rp = q.rowptr.cpu().numpy()
+    return O.nf4_dequant(q.packed.cpu().numpy(), q.absmax.cpu().numpy(), q.marlin_layout, "float32",
+                         rp, q.col.cpu().numpy(), q.val.cpu().numpy(), blocksize=bs)
+
+
+def _check(y, x, w, had, bias, dt):
+    xr = O.rotate_blocks(x.float().cpu().numpy(), had) if had else x.float().cpu().numpy()
+    ref = torch.from_numpy(xr.astype(np.float64)).cuda() @ torch.from_numpy(w.astype(np.float64)).cuda().t()
+    if bias is not None:
+        ref = ref + bias.double()
+    rel = ((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).max().item()  # the worst row
+    assert rel <= (1e-3 if dt == "float16" else 5e-3), rel
+
+
+@pytest.mark.parametrize("m,n,k,had,ratio,marlin,dt,bs", [
+    (17, 128, 1024, 128, 0.01, True, "float16", 64),
+    (32, 129, 64, 64, 0.05, False, "bfloat16", 64),     # one chunk
+    (33, 1000, 1088, 64, 0.01, True, "float16", 32),    # 17 chunks, 32-blocks
+    (64, 3072, 3072, 512, 0.005, True, "float16", 64),
+    (65, 640, 2112, 32, 0.02, False, "float16", 64),    # 33 chunks
+    (96, 5120, 1024, 128, 0.005, True, "bfloat16", 64),
+    (97, 1537, 1024, 0, 0.0, True, "float16", 64),      # two chunks a stage, 4 row tiles
+    (129, 384, 1344, 0, 0.0, False, "float16", 64),     # one chunk a stage, 3 + 3 row tiles
+    (160, 2048, 2048, 256, 0.0, True, "bfloat16", 64),
+    (255, 129, 3072, 2, 0.01, True, "float16", 64),     # few tiles: any row count
+    (257, 77, 4096, 128, 0.01, False, "float16", 64),   # two row blocks
+    (511, 33, 6144, 0, 0.01, True, "float16", 128),
+])
+def test_mid_nf4(hip, m, n, k, had, ratio, marlin, dt, bs):
+    q, _ = _nf4(n, k, had, ratio, marlin, bs)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, generator=g, device="cuda").to(DT[dt])
+    x[m - 1] *= 1000.0  # rows of very different size
+    x[0] *= 1e-3
+    bias = torch.randn(n, generator=g, device="cuda")
+    col, val = q.outliers()
+    y = K.batched_w4a16_gemm(x, q.packed, q.absmax, None, col, val, marlin, codebook="nf4", group_size=bs,
+                             hadamard_block=had, outlier_rowptr=q.rowptr if col is not None else None, bias=bias)
+    _check(y, x, _dense(q, bs), had, bias, dt)
+
+
+@pytest.mark.parametrize("m,n,k,n_out,marlin,dt", [
+    (17, 256, 96 * 2, 3, True, "float16"), (40, 1001, 2112, 20, False, "bfloat16"), (96, 3072, 3072, 30, True, "float16"),
+    (160, 640, 1024, 0, True, "float16"), (300, 99, 2048, 7, True, "float16")])
+def test_mid_format_a(hip, m, n, k, n_out, marlin, dt):
+    rng = np.random.default_rng(m + n)
+    qc = rng.integers(0, 16, (n, k)).astype(np.uint8)  # codes under the outlier columns are not zero
+    z = rng.integers(0, 16, (n, k // 32)).astype(np.uint8)
+    s = (rng.random((n, k // 32)) * 0.01 + 0.001).astype(np.float16)
+    packed = O.pack_nibbles(qc, marlin)
+    w = (qc.astype(np.float32) - np.repeat(z, 32, 1)) * np.repeat(s.astype(np.float32), 32, 1)
+    idx = np.sort(rng.permutation(k)[:n_out]) if n_out else None
+    ow = None
+    if n_out:
+        ow = torch.from_numpy((rng.standard_normal((n, n_out)) * 0.2).astype(np.float32)).to(DT[dt]).cuda()
+        w[:, idx] = ow.float().cpu().numpy()
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, generator=g, device="cuda").to(DT[dt])
+    y = K.batched_w4a16_gemm(x, torch.from_numpy(packed).cuda(), torch.from_numpy(s).cuda(), torch.from_numpy(z).cuda(),
+                             torch.from_numpy(idx).cuda() if n_out else None, ow, marlin)
+    _check(y, x, w, 0, None, dt)
+
+
+def test_mid_strides_alignment_and_workspace(hip):
+    """The C entry with x and out rows padded and x off 16-byte alignment; a workspace that holds only
+    the 256-row-tile GEMM's buffers still runs (that GEMM)."""
+    m, n, k = 50, 333, 1024
+    q, had = _nf4(n, k, 128, 0.01, True)
+    ops = K.QWeightOperands(q.packed, q.absmax, None, k, codebook="nf4", hadamard_block=128, marlin_layout=True,
+                            outlier_idx=q.col, outlier_w=q.val, outlier_rowptr=q.rowptr)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    xb = torch.randn(m, k + 9, generator=g, device="cuda").half()
+    out = torch.full((m, n + 3), 7.0, device="cuda", dtype=torch.float16)
+    need = hip.spectra_w4a16_gemm_workspace(ops.ptr(), m, L.F16)
+    stream = torch.cuda.current_stream().cuda_stream
+    small = next(b for b in range(1 << 16, need, 4096) if b >= m * k * 2 + (1 << 17))
+    for off, size in ((1, need), (0, need), (0, min(small, need - 1))):
+        x = xb[:, off:off + k]
+        ws = torch.empty(size, device="cuda", dtype=torch.uint8)
+        st = hip.spectra_w4a16_gemm(ops.ptr(), x.data_ptr(), xb.stride(0), m, L.F16, out.data_ptr(), out.stride(0),
+                                    ws.data_ptr(), size, stream)
+        if st == L.ERR_WORKSPACE and size < need:
+            continue  # (also smaller than that GEMM needs: refused, nothing launched)
+        assert st == 0
+        _check(out[:, :n], x, _dense(q), 128, None, "float16")
+        assert bool((out[:, n:] == 7.0).all())
