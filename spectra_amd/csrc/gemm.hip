@@ -6,9 +6,9 @@
 //    fp16 rounding.  The row is stored in packed-byte pair order: position 2 b + h holds
 //    the element that nibble h of packed byte b multiplies, so a decoded byte (an fp16
 //    code pair) and the activations it meets sit at the same positions.
-// 2. gemm_outlier_lists_kernel (when the weight has outliers): each group of 16 weight rows'
-//    CSR entries / outlier columns bucketed by K-step, with each entry's position in the
-//    decoded LDS tile precomputed.
+// 2. gemm_outlier_lists (when the weight has outliers; further workgroups of the same launch):
+//    each group of 16 weight rows' CSR entries / outlier columns bucketed by K-step, with each
+//    entry's position in the decoded LDS tile precomputed.
 // 3. gemm_kernel<FMT, BN>: a 256 x BN output tile per workgroup, K step 32, 8 waves of
 //    128 x BN/4 (v_mfma_f32_32x32x16_f16, fp32 accumulators, two waves per SIMD).  Each step
 //    one thread decodes half (BN = 256) or a quarter (BN = 128) of one weight row's 16-byte
@@ -38,7 +38,6 @@ constexpr int kRowH = 32;         // fp16 per LDS tile row (64 bytes, four 16-by
 constexpr int kPrepThreads = 256;
 constexpr int kGLut = 65536;      // lane-replicated nibble-pair LUT at LDS address 0
 constexpr int kOGroup = 16;       // weight rows per outlier step list
-constexpr int kOListThreads = 256;
 
 // 16-byte chunk c of tile row r sits at chunk c ^ tile_swz(r): with 64-byte rows, every
 // 8-lane (32 banks) or 16-lane (64 banks) phase of the tile stores (two or four lanes per
@@ -46,6 +45,103 @@ constexpr int kOListThreads = 256;
 // distinct banks.  The mask takes rows' bits 1..3 only, so rows 32 apart share it.
 __device__ __forceinline__ int tile_swz(int r) {
   return (((r >> 1) ^ (r >> 2)) & 1) | ((((r >> 1) ^ (r >> 3)) & 1) << 1);
+}
+
+// ---------------------------------------------------------------------------
+// outlier step lists
+// ---------------------------------------------------------------------------
+// Outlier step lists for the GEMM, one workgroup per group of kOGroup weight rows: the
+// group's entries (CSR, or the outlier columns of every row) bucketed by K-step with a
+// counting sort in LDS.  ostart[g][s] = first entry of step s (s = 0 .. KS, the last = the
+// group's end), oent[e] = (fp16 index inside the group's 16 LDS tile rows, swizzle applied)
+// << 16 | fp16 value bits -- the tile rows of a group share their swizzle pattern modulo 16,
+// so the position is known here.  The order inside a step is arbitrary: each entry owns its
+// position in the tile.
+struct OListArgs {
+  const int32_t* rowptr;
+  const int32_t* ccol;
+  const uint16_t* cval;
+  const int64_t* oidx;
+  const void* ow;
+  int64_t ldow;
+  int okind, ow_dt, n_out, n;
+  int groups;  // 0: no lists
+  int32_t* ostart;
+  uint32_t* oent;
+};
+
+// cnt: [KS + 1] counts, then cursors
+__device__ __forceinline__ void gemm_outlier_lists(const OListArgs& o, int g, int KS, int marlin, int32_t* cnt) {
+  __shared__ int32_t rp[kOGroup + 1];
+  __shared__ int32_t wtot[kPrepThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int n_out = o.n_out;
+  const bool csr = o.okind == SPECTRA_OUTLIERS_CSR;
+  const int r0 = g * kOGroup, nr = min(kOGroup, o.n - r0);
+  // the group's entries are [rp[0], rp[nr]), row r's [rp[r], rp[r + 1]) (the outlier columns
+  // of every row for Format A: n_out per row)
+  if (tid <= nr) rp[tid] = csr ? o.rowptr[r0 + tid] : (r0 + tid) * n_out;
+  for (int t = tid; t <= KS; t += kPrepThreads) cnt[t] = 0;
+  __syncthreads();
+  const int base = rp[0], total = rp[nr] - base;
+  // entry el of the group: its row, column and fp16 value (entries in parallel, no per-row chain)
+  auto entry = [&](int el, int& r, int& c, uint32_t& v) __attribute__((always_inline)) {
+    if (csr) {
+      const int e = base + el;
+      r = 0;
+#pragma unroll
+      for (int q = 1; q < kOGroup; ++q) r += (q < nr && rp[q] <= e) ? 1 : 0;
+      c = o.ccol[e];
+      v = o.cval[e];
+    } else {
+      r = el / n_out;
+      const int jj = el - r * n_out;
+      c = (int)o.oidx[jj];
+      v = f2h(load_elem(o.ow, (int64_t)(r0 + r) * o.ldow + jj, o.ow_dt));
+    }
+  };
+  for (int el = tid; el < total; el += kPrepThreads) {
+    int r, c;
+    uint32_t v;
+    entry(el, r, c, v);
+    if ((unsigned)c < (unsigned)(KS * kBK)) atomicAdd(&cnt[c / kBK], 1);  // (columns outside K: dropped)
+  }
+  __syncthreads();
+  // exclusive scan of cnt[0, KS): thread t owns a run of `per` consecutive steps
+  const int per = (KS + kPrepThreads - 1) / kPrepThreads;
+  const int lo = min(tid * per, KS), hi = min(lo + per, KS);
+  int run = 0;
+  for (int t = lo; t < hi; ++t) run += cnt[t];
+  int inc = run;  // inclusive scan over the wave
+  for (int d = 1; d < 64; d <<= 1) {
+    const int v = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += v;
+  }
+  if (lane == 63) wtot[wv] = inc;
+  __syncthreads();
+  int pre = inc - run;
+  for (int w = 0; w < wv; ++w) pre += wtot[w];
+  int32_t* og = o.ostart + (int64_t)g * (KS + 1);
+  for (int t = lo; t < hi; ++t) {
+    const int c = cnt[t];
+    cnt[t] = pre;  // cursor
+    og[t] = base + pre;
+    pre += c;
+  }
+  if (tid == kPrepThreads - 1) og[KS] = base + pre;  // the last thread's runs end at KS
+  __syncthreads();
+  for (int el = tid; el < total; el += kPrepThreads) {
+    int r, c;
+    uint32_t v;
+    entry(el, r, c, v);
+    if ((unsigned)c >= (unsigned)(KS * kBK)) continue;
+    const int pos = atomicAdd(&cnt[c / kBK], 1);
+    const int cs = c % kBK;
+    const int jb = marlin ? (cs & 15) : (cs >> 1), h = marlin ? (cs >> 4) : (cs & 1);
+    const int e2 = 2 * jb + h;  // fp16 index in the step's decoded row (packed-byte pair order)
+    const int off = r * kRowH + 8 * ((e2 >> 3) ^ tile_swz(r)) + (e2 & 7);
+    o.oent[base + pos] = ((uint32_t)off << 16) | v;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -65,14 +161,25 @@ constexpr int kPrepMaxU = 16;  // K <= 256 * 8 * 16 = 32768
 // With no row-wide scale to find, blockIdx.y then picks a segment of kPrepThreads * 8 * kPrepU
 // elements of the row (a multiple of every Hadamard block size), so a long row spreads over
 // several workgroups; the scaled mode runs with gridDim.y = 1 (the whole row).
+//
+// The first ol.groups workgroups (scaled mode only) build the outlier step lists: neither job
+// fills the chip (200 rows and 192 groups at N x K = 3072 x 8192), each is a chain of dependent
+// loads, and neither needs the other, so one launch hides the shorter behind the longer and
+// saves a gap: 200 rows of that layer 47.6 -> 42.5 us, 130 rows of Format A
+// 8192 x 3072 with 1% outlier columns 42.0 -> 39.2 us.
 template <int kPrepU>
 __global__ void __launch_bounds__(kPrepThreads) gemm_prep_kernel(const void* __restrict__ a, int64_t lda, int dt,
                                                                   int k, int log_had, float div, int marlin, int vec,
                                                                   uint16_t* __restrict__ a16,
-                                                                  int32_t* __restrict__ fexp, int raw_dt) {
+                                                                  int32_t* __restrict__ fexp, int raw_dt,
+                                                                  const OListArgs ol) {
   extern __shared__ float fs[];  // [k] fp32 (the 1024-block stage), then [k] fp16 (pair-order write)
   __shared__ float wmax[kPrepThreads / 64];
-  const int64_t row = blockIdx.x;
+  if ((int)blockIdx.x < ol.groups) {
+    gemm_outlier_lists(ol, blockIdx.x, k / kBK, marlin, (int32_t*)fs);
+    return;
+  }
+  const int64_t row = (int)blockIdx.x - ol.groups;
   const int tid = threadIdx.x;
   const int64_t seg0 = (int64_t)blockIdx.y * (kPrepThreads * 8 * kPrepU);  // first element
   const int n8 = (int)min((int64_t)k - seg0, (int64_t)kPrepThreads * 8 * kPrepU) >> 3;
@@ -222,10 +329,11 @@ int gemm_prep_rotate(const void* a, int64_t lda, int64_t m, int dt, int k, int h
   if (st != SPECTRA_OK) return st;
   const int vec = (reinterpret_cast<uintptr_t>(a) % 16) == 0 && lda % 8 == 0;
   const int marl = 0, raw_dt = dt;
+  OListArgs ol = {};
   const int seg = kPrepThreads * 8 * 2, nseg = (k + seg - 1) / seg;
   const size_t prep_lds = (size_t)seg * (had > 512 ? 4 : 2);
   void* pargs[] = {(void*)&a, (void*)&lda, (void*)&dt, (void*)&k, (void*)&log_had, (void*)&div, (void*)&marl,
-                   (void*)&vec, (void*)&a16, (void*)&fexp, (void*)&raw_dt};
+                   (void*)&vec, (void*)&a16, (void*)&fexp, (void*)&raw_dt, (void*)&ol};
   SPECTRA_HIP_CHECK(hipLaunchKernel(prep, dim3((unsigned)m, (unsigned)nseg), dim3(kPrepThreads), pargs, prep_lds, s));
   SPECTRA_HIP_CHECK(hipGetLastError());
   return SPECTRA_OK;
@@ -256,7 +364,7 @@ struct GemmParams {
   int gshift, marlin, okind, n_out, ow_dt, bias_dt, act_dt;
   int ksplit, ksteps;  // K splits (blockIdx.z) and kBK-steps per split
   float* part;         // ksplit > 1: fp32 partials [ksplit][m][n]
-  // outlier step lists (gemm_outlier_lists_kernel): ostart[g][s] = first entry of row
+  // outlier step lists (gemm_outlier_lists): ostart[g][s] = first entry of row
   // group g in K-step s (s = 0 .. K / kBK, the last = the group's end); oent = entries
   const int32_t* ostart;
   const uint32_t* oent;
@@ -602,90 +710,6 @@ __global__ void __launch_bounds__(kRedThreads) splitk_reduce_kernel(const float*
   }
 }
 
-// Outlier step lists for the GEMM, one workgroup per group of kOGroup weight rows: the
-// group's entries (CSR, or the outlier columns of every row) bucketed by K-step with a
-// counting sort in LDS.  ostart[g][s] = first entry of step s (s = 0 .. KS, the last = the
-// group's end), oent[e] = (fp16 index inside the group's 16 LDS tile rows, swizzle applied)
-// << 16 | fp16 value bits -- the tile rows of a group share their swizzle pattern modulo 16,
-// so the position is known here.  The order inside a step is arbitrary: each entry owns its
-// position in the tile.
-__global__ void __launch_bounds__(kOListThreads) gemm_outlier_lists_kernel(
-    int okind, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ ccol,
-    const uint16_t* __restrict__ cval, const int64_t* __restrict__ oidx, const void* __restrict__ ow,
-    int64_t ldow, int ow_dt, int n_out, int n, int KS, int marlin, int32_t* __restrict__ ostart,
-    uint32_t* __restrict__ oent) {
-  extern __shared__ int32_t cnt[];  // [KS + 1]: counts, then cursors
-  __shared__ int32_t rp[kOGroup + 1];
-  __shared__ int32_t wtot[kOListThreads / 64];
-  const int g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const bool csr = okind == SPECTRA_OUTLIERS_CSR;
-  const int r0 = g * kOGroup, nr = min(kOGroup, n - r0);
-  // the group's entries are [rp[0], rp[nr]), row r's [rp[r], rp[r + 1]) (the outlier columns
-  // of every row for Format A: n_out per row)
-  if (tid <= nr) rp[tid] = csr ? rowptr[r0 + tid] : (r0 + tid) * n_out;
-  for (int t = tid; t <= KS; t += kOListThreads) cnt[t] = 0;
-  __syncthreads();
-  const int base = rp[0], total = rp[nr] - base;
-  // entry el of the group: its row, column and fp16 value (entries in parallel, no per-row chain)
-  auto entry = [&](int el, int& r, int& c, uint32_t& v) __attribute__((always_inline)) {
-    if (csr) {
-      const int e = base + el;
-      r = 0;
-#pragma unroll
-      for (int q = 1; q < kOGroup; ++q) r += (q < nr && rp[q] <= e) ? 1 : 0;
-      c = ccol[e];
-      v = cval[e];
-    } else {
-      r = el / n_out;
-      const int jj = el - r * n_out;
-      c = (int)oidx[jj];
-      v = f2h(load_elem(ow, (int64_t)(r0 + r) * ldow + jj, ow_dt));
-    }
-  };
-  for (int el = tid; el < total; el += kOListThreads) {
-    int r, c;
-    uint32_t v;
-    entry(el, r, c, v);
-    if ((unsigned)c < (unsigned)(KS * kBK)) atomicAdd(&cnt[c / kBK], 1);  // (columns outside K: dropped)
-  }
-  __syncthreads();
-  // exclusive scan of cnt[0, KS): thread t owns a run of `per` consecutive steps
-  const int per = (KS + kOListThreads - 1) / kOListThreads;
-  const int lo = min(tid * per, KS), hi = min(lo + per, KS);
-  int run = 0;
-  for (int t = lo; t < hi; ++t) run += cnt[t];
-  int inc = run;  // inclusive scan over the wave
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += v;
-  }
-  if (lane == 63) wtot[wv] = inc;
-  __syncthreads();
-  int pre = inc - run;
-  for (int w = 0; w < wv; ++w) pre += wtot[w];
-  int32_t* og = ostart + (int64_t)g * (KS + 1);
-  for (int t = lo; t < hi; ++t) {
-    const int c = cnt[t];
-    cnt[t] = pre;  // cursor
-    og[t] = base + pre;
-    pre += c;
-  }
-  if (tid == kOListThreads - 1) og[KS] = base + pre;  // the last thread's runs end at KS
-  __syncthreads();
-  for (int el = tid; el < total; el += kOListThreads) {
-    int r, c;
-    uint32_t v;
-    entry(el, r, c, v);
-    if ((unsigned)c >= (unsigned)(KS * kBK)) continue;
-    const int pos = atomicAdd(&cnt[c / kBK], 1);
-    const int cs = c % kBK;
-    const int jb = marlin ? (cs & 15) : (cs >> 1), h = marlin ? (cs >> 4) : (cs & 1);
-    const int e2 = 2 * jb + h;  // fp16 index in the step's decoded row (packed-byte pair order)
-    const int off = r * kRowH + 8 * ((e2 >> 3) ^ tile_swz(r)) + (e2 & 7);
-    oent[base + pos] = ((uint32_t)off << 16) | v;
-  }
-}
-
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // tile plan: 256 x 256 tiles once there are at least 64 of them (twice the MFMA work per
@@ -819,12 +843,6 @@ extern "C" int spectra_w4a16_gemm(const spectra_qweight_t* w, const void* a, int
   const int vec = (reinterpret_cast<uintptr_t>(a) % 16) == 0 && lda % 8 == 0;
   const int kk32 = (int)w->k, marl = w->marlin_layout ? 1 : 0;
   const size_t prep_lds = (size_t)w->k * (had > 512 ? 4 : 2);
-  const int scaled = -1;  // per-row power-of-two scale, fp16
-  void* pargs[] = {(void*)&a, (void*)&lda, (void*)&act_dtype, (void*)&kk32, (void*)&log_had, (void*)&div,
-                   (void*)&marl, (void*)&vec, (void*)&a16, (void*)&fexp, (void*)&scaled};
-  SPECTRA_HIP_CHECK(hipLaunchKernel(prep, dim3((unsigned)m), dim3(kPrepThreads), pargs, prep_lds, s));
-  SPECTRA_HIP_CHECK(hipGetLastError());
-
   GemmParams p;
   p.a16 = a16; p.fexp = fexp;
   p.packed = w->packed; p.ldp = w->packed_stride;
@@ -851,6 +869,7 @@ extern "C" int spectra_w4a16_gemm(const spectra_qweight_t* w, const void* a, int
   // outlier step lists (after the partials in the workspace), built for this call
   const int64_t nent = outlier_entries(w);
   const int KS = (int)(w->k / kBK);
+  OListArgs ol = {};
   p.ogroups = (int)((w->n + kOGroup - 1) / kOGroup);
   if (nent > 0) {
     if (nent >= (int64_t(1) << 31)) return fail(SPECTRA_ERR_UNSUPPORTED, "the GEMM family serves < 2^31 outlier entries");
@@ -860,16 +879,20 @@ extern "C" int spectra_w4a16_gemm(const spectra_qweight_t* w, const void* a, int
     uint32_t* oent = (uint32_t*)(lists + align256((size_t)p.ogroups * (size_t)(KS + 1) * 4));
     p.ostart = ostart;
     p.oent = oent;
-    hipLaunchKernelGGL(gemm_outlier_lists_kernel, dim3((unsigned)p.ogroups), dim3(kOListThreads),
-                       (size_t)(KS + 1) * 4, s, p.okind, w->csr_rowptr, w->csr_col, w->csr_val, w->outlier_idx,
-                       w->outlier_w, w->outlier_w_stride, w->outlier_w_dtype, (int)w->num_outliers, (int)w->n, KS,
-                       p.marlin, ostart, oent);
-    SPECTRA_HIP_CHECK(hipGetLastError());
+    ol.rowptr = w->csr_rowptr; ol.ccol = w->csr_col; ol.cval = w->csr_val;
+    ol.oidx = w->outlier_idx; ol.ow = w->outlier_w; ol.ldow = w->outlier_w_stride;
+    ol.okind = p.okind; ol.ow_dt = w->outlier_w_dtype; ol.n_out = (int)w->num_outliers; ol.n = (int)w->n;
+    ol.groups = p.ogroups; ol.ostart = ostart; ol.oent = oent;
   } else {
     p.okind = SPECTRA_OUTLIERS_NONE;
     p.ostart = (const int32_t*)a16;  // readable dummies: the kernel reads index 0 and 1 only
     p.oent = (const uint32_t*)a16;
   }
+  const int scaled = -1;  // per-row power-of-two scale, fp16
+  void* pargs[] = {(void*)&a, (void*)&lda, (void*)&act_dtype, (void*)&kk32, (void*)&log_had, (void*)&div,
+                   (void*)&marl, (void*)&vec, (void*)&a16, (void*)&fexp, (void*)&scaled, (void*)&ol};
+  SPECTRA_HIP_CHECK(hipLaunchKernel(prep, dim3((unsigned)(m + ol.groups)), dim3(kPrepThreads), pargs, prep_lds, s));
+  SPECTRA_HIP_CHECK(hipGetLastError());
   const size_t lds = (size_t)kGLut + (size_t)2 * (kBM + BN) * kRowH * 2 + kBM * 4;
   dim3 grid((unsigned)g.nt, (unsigned)g.mt, (unsigned)g.ksplit);
   const void* kern;
