@@ -53,34 +53,46 @@ __global__ void __launch_bounds__(kDqThreads) scatter_csr_kernel(spectra_qweight
     store_elem(out, row * ldo + w.csr_col[e], out_dt, h2f(w.csr_val[e]));
 }
 
-// f2bf without a branch (same bits: round to nearest even, NaN quieted)
-__device__ __forceinline__ uint32_t f2bf_sel(float f) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, f);
-  const uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-  return (u & 0x7fffffffu) > 0x7f800000u ? ((u >> 16) | 0x40u) : r;
+typedef float dq_f2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 dq_b2_t __attribute__((ext_vector_type(2)));
+
+// two f2bf in one instruction (round to nearest even, NaN quieted: the same bits for every float)
+__device__ __forceinline__ uint32_t f2bf_pair(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(dq_f2_t{lo, hi}, dq_b2_t));
 }
 
 // Row dequant at HBM rate (the prefill path materialises whole weights with it).  One wave per
-// (row, segment of segc 32-element runs, segc <= kDqSegChunks a whole number of passes chosen by
+// (row, segment of segc 32-element runs, segc <= kSegRuns a whole number of passes chosen by
 // the host so that the grid holds about kDqWaves waves); in a pass over a block of 64 kE elements
 // lane l owns the kE consecutive outputs kE l .. kE l + kE - 1 (kE = 8 for 16-bit, 4 for
 // fp32 outputs), so every store instruction of the wave writes 1 KB contiguously.  In both
 // nibble orders the 16 bytes of run c hold elements 32 c .. 32 c + 31 under one scale (group
 // size a multiple of 32): with the marlin pairs (k, k + 16) a lane reads kE bytes and takes
 // their low (first half of the run) or high nibbles, in the natural order kE / 2 bytes and
-// both nibbles.  All of a segment's loads are issued before the first decode.  The NF4 codes
-// come from a 16-entry LDS table.  Same values and roundings as dequant_kernel.  After the
-// segment's dense stores have completed (the wave waits on its store counter; the fence keeps
-// the compiler from moving stores across), the same wave stores the row's outliers that fall
-// in its segment over them, so they land last.
-constexpr int kDqSegChunks = 224;  // at most 7168 elements per segment
+// both nibbles.  All of a segment's loads (packed bytes, scales, outlier
+// entries) are issued before the first decode.  The NF4 codes come from a 16-entry LDS table.  Same
+// values and roundings as dequant_kernel.  A pass's outliers are written over its rounded values in
+// the wave's 1 KB LDS slot, which all 64 lanes do (a partial pass too: an idle lane may hold an
+// entry), and the whole lines then go out once; only entries past the kDqPre * 64 that the wave holds
+// are stored over the row in memory, after the segment's dense stores have completed (the wave waits
+// on its store counter; the fence keeps the compiler from moving stores across).
+// What bounds it: the stores' bandwidth on large weights, the chain row pointer -> entries -> stores
+// on small ones.  fp16 / bf16, 0.5% outliers, us a call in a graph, with scales loaded per pass, the
+// outliers all stored to memory and bf16 rounded in integer arithmetic -> now: 16384 x 3072 25.8 /
+// 30.6 -> 23.4 / 23.0 (5.5 TB/s), 5120 x 3072 14.4 / 16.3 -> 11.8 / 11.7, 3072 x 8192 16.2 / 19.1 ->
+// 15.3 / 14.9, 14336 x 4096 29.3 / 33.1 -> 27.2 / 26.6.
 constexpr int64_t kDqWaves = 12288;  // 48 waves per CU on 256 CUs
 constexpr int kDqPre = 2;            // outlier entries preloaded per lane
 
 template <int kOut, bool kMarlin>
 struct DqShape {
   static constexpr int kE = kOut == SPECTRA_F32 ? 4 : 8;   // outputs per lane per pass
-  static constexpr int kPasses = kDqSegChunks * 32 / (64 * kE);
+  // runs of a segment at most: 4096 elements (8 passes) for 16-bit outputs, 7168 for fp32
+  static constexpr int kSegRuns = kOut == SPECTRA_F32 ? 224 : 128;
+  static constexpr int kPasses = kSegRuns * 32 / (64 * kE);
+  // 16-bit outputs: the scales of every pass are loaded with its bytes (62 VGPRs at most).  With
+  // fp32's twice as many passes that took 121 VGPRs, and Format A 14336 x 4096 went from 44 to 62 us
+  static constexpr bool kScalesAhead = kOut != SPECTRA_F32;
   static constexpr int kBytes = kMarlin ? kE : kE / 2;      // packed bytes per lane per pass
 };
 
@@ -106,25 +118,36 @@ __global__ void __launch_bounds__(kDqThreads) dequant_rows_kernel(spectra_qweigh
   typedef DqShape<kOut, kMarlin> S;
   static_assert(!kRot || S::kE == 8, "the rotated rows are 16-bit outputs");
   __shared__ float code[16];
-  __shared__ __align__(16) float stage[kRot ? kDqThreads / 64 : 1][kRot ? 512 : 4];
+  __shared__ __align__(16) float stage[kDqThreads / 64][kRot ? 512 : 256];  // a wave's pass
   if (threadIdx.x < 16) code[threadIdx.x] = nf4_code_f32((int)threadIdx.x);
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  const int64_t wid = (int64_t)blockIdx.x * (kDqThreads / 64) + (threadIdx.x >> 6);
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t wid = (int64_t)blockIdx.x * (kDqThreads / 64) + wv;
   const int64_t row = wid / nseg;
   if (row >= w.n) return;
   const int nch = (int)(w.k >> 5);
   const int c0 = (int)(wid - row * nseg) * segc;
   const int e_end = 32 * (min(nch, c0 + segc) - c0);  // elements of this segment
-  const int gch = kAsym ? 1 : w.group_size >> 5;              // runs per scale group
+  const int gsh = kAsym ? 0 : __builtin_ctz((unsigned)w.group_size) - 5;  // runs per scale group, log2
   const uint8_t* prow = w.packed + row * w.packed_stride + 16 * (int64_t)c0;
   uint64_t qb[S::kPasses];
+  uint16_t sb[S::kPasses];
+  uint8_t zb[S::kPasses];
+  const uint16_t* srow = w.scales + row * w.scales_stride;
+  auto scale = [&](int b, int o) __attribute__((always_inline)) {
+    sb[b] = srow[(c0 + (o >> 5)) >> gsh];
+    if (kAsym) zb[b] = w.zeros[row * w.zeros_stride + c0 + (o >> 5)];
+  };
 #pragma unroll
   for (int b = 0; b < S::kPasses; ++b) {
-    const int o = 64 * S::kE * b + S::kE * lane;  // first element of the lane's outputs
+    // first element of the lane's outputs (past a last, partial pass: its last ones again)
+    const int o = min(64 * S::kE * b + S::kE * lane, e_end - S::kE);
     const int e0 = o & 31;
-    if (o < e_end)
+    if (64 * S::kE * b < e_end) {
       qb[b] = load_bytes<S::kBytes>(prow + 16 * (o >> 5) + (kMarlin ? (e0 & 15) : (e0 >> 1)));
+      if (S::kScalesAhead) scale(b, o);
+    }
   }
   // the first kDqPre * 64 outlier entries of the row (column, value), loaded with the weights so
   // that the tail below only filters and stores them
@@ -154,11 +177,12 @@ __global__ void __launch_bounds__(kDqThreads) dequant_rows_kernel(spectra_qweigh
   }
 #pragma unroll
   for (int b = 0; b < S::kPasses; ++b) {
+    if (64 * S::kE * b >= e_end) break;
     const int o = 64 * S::kE * b + S::kE * lane;
-    if (o >= e_end) break;
-    const int c = c0 + (o >> 5), e0 = o & 31;
-    const float s = h2f(w.scales[row * w.scales_stride + c / gch]);
-    const float z = kAsym ? (float)w.zeros[row * w.zeros_stride + c] : 0.0f;
+    const int e0 = o & 31;
+    if (!S::kScalesAhead) scale(b, min(o, e_end - S::kE));
+    const float s = h2f(sb[b]);
+    const float z = kAsym ? (float)zb[b] : 0.0f;
     float v[S::kE];
 #pragma unroll
     for (int i = 0; i < S::kE; ++i) {
@@ -177,23 +201,26 @@ __global__ void __launch_bounds__(kDqThreads) dequant_rows_kernel(spectra_qweigh
     if constexpr (kRot) {
       // the pass's dense values and its outliers through the wave's LDS slot (one wave:
       // in-order LDS, the wait and the memory clobber keep every read after every write)
-      float* st = stage[threadIdx.x >> 6];
+      // (a lane's first four values in the first half of the slot, the others in the second:
+      // 16-byte accesses at a 16-byte stride)
+      float* st = stage[wv];
+      auto at = [](int e) { return ((e & 4) << 6) + ((e >> 3) << 2) + (e & 3); };
       const int64_t pk0 = 32 * (int64_t)c0 + 64 * S::kE * b;  // first column of the pass
-      *(float4*)&st[8 * lane] = make_float4(v[0], v[1], v[2], v[3]);
-      *(float4*)&st[8 * lane + 4] = make_float4(v[4], v[5], v[6], v[7]);
+      *(float4*)&st[4 * lane] = make_float4(v[0], v[1], v[2], v[3]);
+      *(float4*)&st[256 + 4 * lane] = make_float4(v[4], v[5], v[6], v[7]);
 #pragma unroll
       for (int t = 0; t < kDqPre; ++t)
-        if (ocol[t] >= pk0 && ocol[t] < pk0 + 512) st[ocol[t] - pk0] = oval[t];
+        if (ocol[t] >= pk0 && ocol[t] < pk0 + 512) st[at((int)(ocol[t] - pk0))] = oval[t];
       for (int64_t e = e_beg + 64 * kDqPre + lane; e < e_lim; e += 64) {  // rows with more entries
         const int64_t col = w.outlier_kind == SPECTRA_OUTLIERS_CSR ? (int64_t)w.csr_col[e] : w.outlier_idx[e];
         if (col >= pk0 && col < pk0 + 512)
-          st[col - pk0] = w.outlier_kind == SPECTRA_OUTLIERS_CSR
-                              ? h2f(w.csr_val[e])
-                              : load_elem(w.outlier_w, row * w.outlier_w_stride + e, w.outlier_w_dtype);
+          st[at((int)(col - pk0))] = w.outlier_kind == SPECTRA_OUTLIERS_CSR
+                                         ? h2f(w.csr_val[e])
+                                         : load_elem(w.outlier_w, row * w.outlier_w_stride + e, w.outlier_w_dtype);
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       float r[1][8];
-      const float4 ra = *(const float4*)&st[8 * lane], rb = *(const float4*)&st[8 * lane + 4];
+      const float4 ra = *(const float4*)&st[4 * lane], rb = *(const float4*)&st[256 + 4 * lane];
       r[0][0] = ra.x; r[0][1] = ra.y; r[0][2] = ra.z; r[0][3] = ra.w;
       r[0][4] = rb.x; r[0][5] = rb.y; r[0][6] = rb.z; r[0][7] = rb.w;
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot is rewritten by the next pass
@@ -225,24 +252,41 @@ __global__ void __launch_bounds__(kDqThreads) dequant_rows_kernel(spectra_qweigh
         if (kOut == SPECTRA_F16) asm volatile("" : "+v"(v[i]));  // fp32, then fp16
       }
     }
+    uint4 r4;
     if (kOut == SPECTRA_F32) {
-      *(float4*)((float*)out + row * ldo + 32 * (int64_t)c0 + o) = make_float4(v[0], v[1], v[2], v[3]);
+      r4 = make_uint4(__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),
+                      __builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3]));
     } else {
       uint32_t p[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        p[i] = kOut == SPECTRA_BF16 ? f2bf_sel(v[2 * i]) | (f2bf_sel(v[2 * i + 1]) << 16)
+        p[i] = kOut == SPECTRA_BF16 ? f2bf_pair(v[2 * i], v[2 * i + 1])
                                     : (uint32_t)f2h(v[2 * i]) | ((uint32_t)f2h(v[2 * i + 1]) << 16);
-      *(uint4*)((uint16_t*)out + row * ldo + 32 * (int64_t)c0 + o) = make_uint4(p[0], p[1], p[2], p[3]);
+      r4 = make_uint4(p[0], p[1], p[2], p[3]);
     }
+    if (!kRot && e_lim > e_beg) {  // the pass's outliers over its rounded values, in the wave's LDS slot
+      uint8_t* st = (uint8_t*)stage[wv];
+      const int64_t pk0 = 32 * (int64_t)c0 + 64 * S::kE * b;
+      const int64_t pk1 = min(pk0 + 64 * S::kE, 32 * (int64_t)c0 + e_end);
+      *(uint4*)(st + 16 * lane) = r4;
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int t = 0; t < kDqPre; ++t)
+        if (ocol[t] >= pk0 && ocol[t] < pk1) store_elem(st, ocol[t] - pk0, kOut, oval[t]);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      r4 = *(const uint4*)(st + 16 * lane);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot is rewritten by the next pass
+    }
+    if (o >= e_end) continue;  // (a partial pass: these lanes only place outliers)
+    if (kOut == SPECTRA_F32)
+      *(uint4*)((float*)out + row * ldo + 32 * (int64_t)c0 + o) = r4;
+    else
+      *(uint4*)((uint16_t*)out + row * ldo + 32 * (int64_t)c0 + o) = r4;
   }
   const int64_t k0 = 32 * (int64_t)c0, k1 = k0 + e_end;
-  if (!kRot && e_lim > e_beg) {
+  if (!kRot && e_lim > e_beg + 64 * kDqPre) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);
-#pragma unroll
-    for (int t = 0; t < kDqPre; ++t)
-      if (ocol[t] >= k0 && ocol[t] < k1) store_elem(out, row * ldo + ocol[t], out_dt, oval[t]);
     for (int64_t e = e_beg + 64 * kDqPre + lane; e < e_lim; e += 64) {  // rows with more entries
       const int64_t col = w.outlier_kind == SPECTRA_OUTLIERS_CSR ? (int64_t)w.csr_col[e] : w.outlier_idx[e];
       if (col >= k0 && col < k1)
@@ -394,11 +438,11 @@ static int launch_dequant_rows(const spectra_qweight_t* w, void* out, int64_t ld
   spectra_qweight_t wc = *w;
   int odt = out_dtype;
   // segments of whole passes (16 runs for 16-bit outputs, 8 for fp32): enough of them for
-  // about kDqWaves waves, none longer than kDqSegChunks runs
+  // about kDqWaves waves, none longer than kSegRuns
   const int64_t nch = w->k / 32, unit = esz == 4 ? 8 : 16;
   int64_t ns = std::min((nch + unit - 1) / unit, std::max<int64_t>(1, (kDqWaves + w->n - 1) / w->n));
   int64_t sc = ((nch + ns - 1) / ns + unit - 1) / unit * unit;
-  sc = std::min<int64_t>(sc, kDqSegChunks);
+  sc = std::min<int64_t>(sc, esz == 4 ? DqShape<SPECTRA_F32, true>::kSegRuns : DqShape<SPECTRA_F16, true>::kSegRuns);
   int nseg = (int)((nch + sc - 1) / sc), segc = (int)sc;
   int log_had = 0;
   while (rot_had > 1 && (1 << log_had) < rot_had) ++log_had;
