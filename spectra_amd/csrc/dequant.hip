@@ -7,6 +7,7 @@
 #include <cmath>
 
 #include "common.h"
+#include "gemm_prep.h"
 
 namespace spectra {
 
@@ -111,19 +112,45 @@ __device__ __forceinline__ uint64_t load_bytes(const uint8_t* p) {
 // them, back into registers, then the transform (stages 1, 2, 4 in registers, 8 .. 256 across
 // the lanes of a block, as gemm_prep_kernel), the sign and 1 / sqrt(b) in one product, one
 // rounding to the output dtype.  There is no outlier tail.
+//
+// The first ra.wgs workgroups (16-bit outputs, not kRot) rotate the activations of the same prefill
+// call (blocks up to 512): they wait on their own loads and a barrier while the rows stream, and
+// the product needs both.  777 rows through four 3072-wide decoder layers (QKV and gate_up rotate
+// their activations, 5.6 us a launch): 1388 -> 1339 us; 2048 rows of 14336 x 4096 206.5 -> 205.7.
+struct RotateArgs {
+  const void* a;  // activations in the output dtype, row stride lda
+  int64_t lda;
+  uint16_t* a16;
+  int32_t* fexp;
+  int wgs, nseg;  // workgroups (0: no activations), segments of a row
+  int k, log_had, vec;
+  float div;
+};
+constexpr int kRotateU = 2;  // 4096-element segments
+static_assert(kPrepThreads == kDqThreads, "one launch runs both");
+
 template <bool kAsym, int kOut, bool kMarlin, bool kRot>
 __global__ void __launch_bounds__(kDqThreads) dequant_rows_kernel(spectra_qweight_t w, void* __restrict__ out,
                                                                    int64_t ldo, int out_dt, int nseg, int segc,
-                                                                   int log_had, float rot_scale) {
+                                                                   int log_had, float rot_scale,
+                                                                   const RotateArgs ra) {
   typedef DqShape<kOut, kMarlin> S;
   static_assert(!kRot || S::kE == 8, "the rotated rows are 16-bit outputs");
   __shared__ float code[16];
   __shared__ __align__(16) float stage[kDqThreads / 64][kRot ? 512 : 256];  // a wave's pass
+  if constexpr (!kRot && kOut != SPECTRA_F32) {
+    if ((int)blockIdx.x < ra.wgs) {
+      const int sg = blockIdx.x % ra.nseg, row = blockIdx.x / ra.nseg;
+      gemm_prep_row<kRotateU>(ra.a, ra.lda, kOut, ra.k, ra.log_had, ra.div, 0, ra.vec, ra.a16, ra.fexp, kOut, row, sg,
+                              nullptr);
+      return;
+    }
+  }
   if (threadIdx.x < 16) code[threadIdx.x] = nf4_code_f32((int)threadIdx.x);
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t wid = (int64_t)blockIdx.x * (kDqThreads / 64) + wv;
+  const int64_t wid = (int64_t)((int)blockIdx.x - ra.wgs) * (kDqThreads / 64) + wv;
   const int64_t row = wid / nseg;
   if (row >= w.n) return;
   const int nch = (int)(w.k >> 5);
@@ -413,7 +440,7 @@ bool dequant_rows_ok(const spectra_qweight_t* w, const void* out, int64_t ldo, i
 
 // the row kernel's launch; SPECTRA_ERR_UNSUPPORTED (nothing launched) where dequant_rows_ok fails
 static int launch_dequant_rows(const spectra_qweight_t* w, void* out, int64_t ldo, int out_dtype, int rot_had,
-                               hipStream_t s) {
+                               RotateArgs ra, hipStream_t s) {
   if (!dequant_rows_ok(w, out, ldo, out_dtype, rot_had)) return SPECTRA_ERR_UNSUPPORTED;
   const int esz = out_dtype == SPECTRA_F32 ? 4 : 2;
   const bool asym = w->format == SPECTRA_FMT_ASYM_G32;
@@ -449,10 +476,10 @@ static int launch_dequant_rows(const spectra_qweight_t* w, void* out, int64_t ld
   const float div = rot_had > 1 ? (float)std::sqrt((double)rot_had) : 1.0f;
   float rot_scale = 1.0f / div;  // the activation prep's 2^0 / sqrt(b)
   void* args[] = {(void*)&wc, (void*)&out, (void*)&ldo, (void*)&odt, (void*)&nseg, (void*)&segc,
-                  (void*)&log_had, (void*)&rot_scale};
+                  (void*)&log_had, (void*)&rot_scale, (void*)&ra};
   const int64_t waves = w->n * nseg, per_block = kDqThreads / 64;
-  SPECTRA_HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)((waves + per_block - 1) / per_block)), dim3(kDqThreads),
-                                    args, 0, s));
+  SPECTRA_HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)(ra.wgs + (waves + per_block - 1) / per_block)),
+                                    dim3(kDqThreads), args, 0, s));
   SPECTRA_HIP_CHECK(hipGetLastError());
   return SPECTRA_OK;
 }
@@ -462,7 +489,28 @@ static int launch_dequant_rows(const spectra_qweight_t* w, void* out, int64_t ld
 // kernel does not serve the operands (then the activations are rotated instead)
 int w4_dequant_rotated(const spectra_qweight_t* w, void* out, int out_dtype, int had, hipStream_t s) {
   if (out_dtype != SPECTRA_F16 && out_dtype != SPECTRA_BF16) return SPECTRA_ERR_UNSUPPORTED;
-  return launch_dequant_rows(w, out, w->k, out_dtype, had, s);
+  return launch_dequant_rows(w, out, w->k, out_dtype, had, RotateArgs{}, s);
+}
+
+// the prefill library path's operands in one launch: W_eff in the 16-bit dtype of the activations,
+// row stride K, and the m activation rows rotated (blocks of had <= 512) into a16;
+// SPECTRA_ERR_UNSUPPORTED (nothing launched) otherwise
+int w4_dequant_and_rotate(const spectra_qweight_t* w, void* out, int dtype, const void* a, int64_t lda, int64_t m,
+                          uint16_t* a16, int32_t* fexp, hipStream_t s) {
+  const int had = w->hadamard_block;
+  if ((dtype != SPECTRA_F16 && dtype != SPECTRA_BF16) || had > 512) return SPECTRA_ERR_UNSUPPORTED;
+  const int seg = kPrepThreads * 8 * kRotateU;
+  RotateArgs ra;
+  ra.a = a; ra.lda = lda; ra.a16 = a16; ra.fexp = fexp;
+  ra.k = (int)w->k;
+  ra.nseg = (int)((w->k + seg - 1) / seg);
+  if (m * ra.nseg > (int64_t(1) << 24)) return SPECTRA_ERR_UNSUPPORTED;
+  ra.wgs = (int)m * ra.nseg;
+  ra.log_had = 0;
+  while (had > 1 && (1 << ra.log_had) < had) ++ra.log_had;
+  ra.div = had > 1 ? (float)std::sqrt((double)had) : 1.0f;
+  ra.vec = (reinterpret_cast<uintptr_t>(a) % 16) == 0 && lda % 8 == 0;
+  return launch_dequant_rows(w, out, w->k, dtype, 0, ra, s);
 }
 
 }  // namespace spectra
@@ -475,7 +523,7 @@ extern "C" int spectra_w4_dequant(const spectra_qweight_t* w, void* out, int64_t
   SPECTRA_REQUIRE(ldo >= w->k, "out row stride smaller than K");
   SPECTRA_REQUIRE(out_dtype >= SPECTRA_F16 && out_dtype <= SPECTRA_F32, "bad out dtype");
   const hipStream_t s = (hipStream_t)stream;
-  st = launch_dequant_rows(w, out, ldo, (int)out_dtype, 0, s);
+  st = launch_dequant_rows(w, out, ldo, (int)out_dtype, 0, RotateArgs{}, s);
   if (st != SPECTRA_ERR_UNSUPPORTED) return st;
   const int64_t work = w->n * (w->k / 2);
   hipLaunchKernelGGL(dequant_kernel, dim3((unsigned)((work + kDqThreads - 1) / kDqThreads)), dim3(kDqThreads), 0, s,

@@ -35,6 +35,9 @@ int gemm_prep_rotate(const void* a, int64_t lda, int64_t m, int dt, int k, int h
 // dequant.hip: the row dequant's operand check and its rotated rows (W_eff H_b / sqrt(b))
 bool dequant_rows_ok(const spectra_qweight_t* w, const void* out, int64_t ldo, int out_dtype, int rot_had);
 int w4_dequant_rotated(const spectra_qweight_t* w, void* out, int out_dtype, int had, hipStream_t s);
+// ... and W_eff with the rotated activations, one launch (SPECTRA_ERR_UNSUPPORTED: nothing launched)
+int w4_dequant_and_rotate(const spectra_qweight_t* w, void* out, int dtype, const void* a, int64_t lda, int64_t m,
+                          uint16_t* a16, int32_t* fexp, hipStream_t s);
 
 constexpr int64_t kPrefillMinM = 512;
 constexpr size_t kPrefillLtWorkspace = size_t(32) << 20;
@@ -176,9 +179,16 @@ int prefill_launch(const spectra_qweight_t* w, const void* a, int64_t lda, int64
   const uint16_t* a16 = direct_a ? (const uint16_t*)a : (const uint16_t*)(ws + L.a16);
   // (1) W_eff [N][K] in the compute dtype (outliers included; rotated when rot_w), (2) the
   // rotated activations
-  int st = rot_w ? w4_dequant_rotated(w, weff, act_dtype, had, s) : spectra_w4_dequant(w, weff, w->k, act_dtype, s);
-  if (st != SPECTRA_OK) return st;
-  if (!direct_a) {
+  int st = SPECTRA_ERR_UNSUPPORTED;
+  if (!direct_a)  // both in one launch
+    st = w4_dequant_and_rotate(w, weff, act_dtype, a, lda, m, (uint16_t*)(ws + L.a16), (int32_t*)(ws + L.fexp), s);
+  const bool both = st == SPECTRA_OK;
+  if (!both && st != SPECTRA_ERR_UNSUPPORTED) return st;
+  if (!both) {
+    st = rot_w ? w4_dequant_rotated(w, weff, act_dtype, had, s) : spectra_w4_dequant(w, weff, w->k, act_dtype, s);
+    if (st != SPECTRA_OK) return st;
+  }
+  if (!direct_a && !both) {
     st = gemm_prep_rotate(a, lda, m, act_dtype, (int)w->k, w->hadamard_block, (uint16_t*)(ws + L.a16),
                           (int32_t*)(ws + L.fexp), s);
     if (st != SPECTRA_OK) return st;

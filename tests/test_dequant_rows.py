@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import oracle as O
+from spectra_amd import compressor as C
 from spectra_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
@@ -31,3 +32,26 @@ def test_pass_and_segment_edges(hip, k, bs, marlin, out_dt):
                      marlin_layout=marlin, outlier_idx=d["col"], outlier_w=d["val"], outlier_rowptr=d["rowptr"])
     y = y.view(torch.int32 if out_dt == "float32" else torch.int16).cpu().numpy()
     assert np.array_equal(y, np.ascontiguousarray(ref).view(y.dtype))
+
+
+@pytest.mark.parametrize("k,had,off,dt", [(192, 64, 0, torch.float16), (4160, 32, 0, torch.bfloat16),
+                                          (4224, 128, 1, torch.float16), (1024, 512, 0, torch.bfloat16)])
+def test_activations_rotated_in_the_same_launch(hip, k, had, off, dt):
+    """Prompt-size calls that rotate the activations (4 M < N): rows of a partial and of more than one
+    4096-element segment, unaligned rows.  Bound: operands and result rounded to the activations'
+    dtype, u = 2^-11 (fp16) or 2^-8 (bf16) each: rel-L2 <= 3 u."""
+    m, n = 513, 2080
+    g = torch.Generator(device="cuda").manual_seed(k)
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    mask = torch.rand(n, k, generator=g, device="cuda") < 0.01
+    q = C.quantize_nf4(torch.where(mask, w * 10, w).half(), 64, 0, mask, True)
+    buf = torch.randn(m * (k + 8) + 8, generator=g, device="cuda").to(dt)
+    x = buf[off: off + m * (k + 8)].view(m, k + 8)[:, :k]
+    assert not K.prefill_rotates_weights(m, n, k, had)
+    y = K.batched_w4a16_gemm(x, q.packed, q.absmax, None, outlier_idx=q.col, outlier_w=q.val, marlin_layout=True,
+                             codebook="nf4", group_size=64, hadamard_block=had, outlier_rowptr=q.rowptr)
+    dense = O.nf4_dequant(q.packed.cpu().numpy(), q.absmax.cpu().numpy(), True, "float32", q.rowptr.cpu().numpy(),
+                          q.col.cpu().numpy(), q.val.cpu().numpy())
+    ref = torch.from_numpy(O.rotate_blocks(x.float().cpu().numpy(), had)).double() @ torch.from_numpy(dense).double().t()
+    err = (y.double().cpu() - ref).norm() / ref.norm()
+    assert err <= 3 * (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8), err
