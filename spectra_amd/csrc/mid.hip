@@ -454,7 +454,9 @@ __global__ void __launch_bounds__(kMidThreads) mid_kernel(const MidParams p) {
 #pragma unroll
   for (int d = 0; d < ST; ++d) decode(b[0][d], d, 0, 0);
   sload(0, 4);
-  asm volatile("s_barrier" ::: "memory");  // (stage 0 writes over the first quad of a one-stage quad)
+  // stage 0 of a one-stage quad writes over the first quad: its reads have arrived (Format A's
+  // decode, plain arithmetic, may sink past the barrier and with it the wait for them)
+  asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");
   // Stage s: the products of its operands, with the next stage's decoded, its fragments written
   // to the other buffer and the loads of s + 1 + AS (fragments), s + 5 (scales) and the quad UQ (+ 1)
   // ahead issued in between (past the range: its last chunk again).
