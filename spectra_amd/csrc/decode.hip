@@ -820,10 +820,11 @@ __global__ void __launch_bounds__(64 * NW) attend_mfma_kernel(const uint16_t* __
     }
     ms = fmaxf(ms, lane_xor<16>(ms, lane));
     ms = fmaxf(ms, lane_xor<32>(ms, lane));
+    const float me = ms == -INFINITY ? 0.0f : ms;  // no valid row, or scores of -inf only: every e is 0
     float ls = 0.0f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      e[r] = pb + r < n ? __expf(e[r] - ms) : 0.0f;  // (no valid row: ms = -inf, every e 0)
+      e[r] = pb + r < n ? __expf(e[r] - me) : 0.0f;
       ls += e[r];
     }
     ls += lane_xor<16>(ls, lane);
@@ -837,8 +838,8 @@ __global__ void __launch_bounds__(64 * NW) attend_mfma_kernel(const uint16_t* __
       mx = ms;
       l = ls;
     } else {
-      const float mn = fmaxf(mx, ms);  // finite: a later span's workgroup has a whole first one
-      const float fo = __expf(mx - mn), fs = ms == -INFINITY ? 0.0f : __expf(ms - mn);
+      const float mn = fmaxf(mx, ms), mb = mn == -INFINITY ? 0.0f : mn;  // (-inf: both are sums of nothing)
+      const float fo = __expf(mx - mb), fs = __expf(ms - mb);
       l = l * fo + ls * fs;
       mx = mn;
 #pragma unroll

@@ -34,3 +34,19 @@ def test_attend_long(hip, heads, kv, hd, L, positions):
         s = (kd * row[:heads].double()[:, None]).sum(-1) / math.sqrt(hd)
         ref = (torch.softmax(s, -1)[..., None] * vd).sum(1)
         assert (out.double() - ref).abs().max().item() <= 2.0 ** -10 * vd.abs().max().item(), p
+
+
+@pytest.mark.parametrize("L,rows", [(2049, (0, 16)), (9000, (0, 16)), (9000, (4096, 4112)), (9000, (128, 9000))])
+def test_attend_long_infinite_scores(hip, L, rows):
+    """Scores of -inf weigh nothing, also over all 16 rows that a wave takes of a span, in its first
+    span and in a later one.  Bound as above."""
+    heads, kv, hd, p = 2, 1, 128, L - 1
+    g = torch.Generator(device="cuda").manual_seed(L + rows[0])
+    k, v = (torch.randn(kv, L, hd, generator=g, device="cuda").half() for _ in range(2))
+    qkv = torch.randn((heads + 2 * kv) * hd, generator=g, device="cuda").half().abs()
+    k[:, rows[0]:rows[1], 0] = float("-inf")
+    ws = torch.zeros(K.attend_workspace_bytes(heads, hd, L), dtype=torch.uint8, device="cuda")
+    out = K.attend_decode(qkv, torch.tensor([p], device="cuda"), None, None, heads, kv, k, v, ws)
+    s = (k.double() * qkv.view(-1, hd)[:heads].double()[:, None]).sum(-1) / math.sqrt(hd)
+    ref = (torch.softmax(s, -1)[..., None] * v.double()).sum(1)
+    assert (out.double() - ref).abs().max().item() <= 2.0 ** -10 * v.double().abs().max().item()
