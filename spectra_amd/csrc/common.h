@@ -237,7 +237,7 @@ __device__ __forceinline__ float wave_max(float v) {
 // and the fma rounds once, as the reference's add / subtract does).  Partners share their
 // sign before every stage, and the lane's final sign (-1)^(high sides taken) rides on
 // the output scale.
-// (distances 1, 2, 8: one v_fmac_f32_dpp per value, eight per block behind the two wait
+// (distances 1, 2, 7, 8: one v_fmac_f32_dpp per value, eight per block behind the two wait
 // states a DPP source needs after its VALU write)
 #define SPECTRA_PFLY(CTRL, A)                                                          \
   asm volatile("s_nop 1\n"                                                            \
@@ -259,6 +259,7 @@ __device__ __forceinline__ void prep_fly(float (&v)[U][8], float c, int lane) {
   for (int u = 0; u < U; ++u) {
     if constexpr (LB == 1) SPECTRA_PFLY("quad_perm:[1,0,3,2]", v[u]);
     else if constexpr (LB == 2) SPECTRA_PFLY("quad_perm:[2,3,0,1]", v[u]);
+    else if constexpr (LB == 7) SPECTRA_PFLY("row_half_mirror", v[u]);  // (lane ^ 7)
     else if constexpr (LB == 8) SPECTRA_PFLY("row_ror:8", v[u]);
     else {
 #pragma unroll

@@ -192,15 +192,16 @@ __device__ __forceinline__ void mid_entries(const MidSide& en, int k, int marlin
 }
 
 // Workgroups [0, sblocks): block scales and outlier entries; the others: 8 rows (one per wave) x
-// segs 512-k segments (lane l: elements 8 l .. 8 l + 7 of each).  The row scale comes from a bound
-// every workgroup computes from the whole raw row: max |x_rot| <= sqrt(b) max |x|, so |x_rot| 2^F
-// <= 2^15 (fp16 keeps its 11 bits either way); magnitudes are compared as 15-bit integers, two to
-// an instruction (an infinity or a NaN is the largest and takes its own row with it, as any
-// product would).  FWHT stages 1, 2, 4 run in registers, 8 .. 256 across lanes.  Fragments leave
-// through LDS in whole 128-byte lines (8 rows x 16 bytes); the k-major copy in 16-byte pieces.
-template <bool VEC>
-__global__ void __launch_bounds__(kMidPrepThreads) mid_prep_kernel(const uint16_t* __restrict__ a, int64_t lda, int dt,
-                                                                    int m, int k, int log_had, float div, int marlin,
+// segs 512-k segments (lane l: elements 8 l .. 8 l + 7 of each).  The row scale, max |x_rot| 2^F in
+// [2^14, 2^15), is every workgroup's own pass over the whole rotated row: with a bound from the raw row
+// (sqrt(b) max |x|) one large activation cost the small ones up to 4.5 of fp16's octaves.  Without a
+// rotation magnitudes are compared as 15-bit integers, two to an instruction (an infinity or a NaN is
+// the largest and takes its own row with it, as any product would).  FWHT stages 1, 2, 4 run in
+// registers, 8 .. 256 across lanes.  Fragments leave through LDS in whole 128-byte lines (8 rows x
+// 16 bytes); the k-major copy in 16-byte pieces.
+template <bool VEC, int DT>
+__global__ void __launch_bounds__(kMidPrepThreads) mid_prep_kernel(const uint16_t* __restrict__ a, int64_t lda, int m,
+                                                                    int k, int log_had, float div, int marlin,
                                                                     uint16_t* __restrict__ frag,
                                                                     uint16_t* __restrict__ xk, int mp,
                                                                     int32_t* __restrict__ fexp, int sblocks, int segs,
@@ -231,42 +232,14 @@ __global__ void __launch_bounds__(kMidPrepThreads) mid_prep_kernel(const uint16_
     }
     return q;
   };
-  mus2_t mx = {0, 0};
-  for (int e = 8 * lane; e < k; e += 16 * kMidPrepSeg) {  // sixteen loads in flight (past the end: the first again)
-    mu4_t f[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) f[j] = load8(e + kMidPrepSeg * j < k ? e + kMidPrepSeg * j : e);
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        mx = __builtin_elementwise_max(mx, __builtin_bit_cast(mus2_t, f[j][i] & 0x7fff7fffu));
-  }
-  float mr = wave_max(fmaxf(to_f32_16(mx[0], dt), to_f32_16(mx[1], dt)));
-  if (log_had > 0) mr = mr * div * 1.0009765625f;
-  const uint32_t bits = __builtin_bit_cast(uint32_t, mr);
-  const int eb = (int)(bits >> 23);
-  const int E = eb == 0 ? -126 : eb - 127;
-  int F = bits == 0 ? 0 : 14 - E;
-  F = F < -126 ? -126 : (F > 126 ? 126 : F);
-  if (s0 == 0 && lane == 0 && r0 + wv < m) fexp[r0 + wv] = F;
-  const float f2 = __builtin_bit_cast(float, (uint32_t)(F + 127) << 23);
-  // unit of this lane in its 32-run (lane & 3 = q holds elements 8 q .. 8 q + 7): plain order,
-  // elements 8 q ..; Marlin order, the pairs (k, k + 16) for k = 4 d .. 4 d + 3, which the
-  // lanes q and q ^ 2 build from each other's halves (d = 0, 2, 1, 3 for q = 0, 1, 2, 3)
-  const int q = lane & 3;
-  const int d = marlin ? ((q & 1) << 1) | (q >> 1) : q;
-  const int nc = k >> 6, t = r0 >> 5, rl = r0 & 31;
-  for (int sg = s0; sg < min(s0 + segs, nseg); ++sg) {
-    const int k0 = sg * kMidPrepSeg;
-    const mu4_t x = load8(k0 + 8 * lane < k ? k0 + 8 * lane : 0);  // k is a multiple of 64
-    float v[1][8];
+  // eight elements of the row, blockwise transformed but for the sign (returned) and 1 / sqrt(b):
+  // stages 1, 2, 4, ...: (u, v) -> (u + v, u - v) in fp32 (compressor.py:34-39)
+  auto rotate = [&](const mu4_t& x, float (&v)[1][8]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      v[0][2 * i] = to_f32_16((uint16_t)(x[i] & 0xffffu), dt);
-      v[0][2 * i + 1] = to_f32_16((uint16_t)(x[i] >> 16), dt);
+      v[0][2 * i] = to_f32_16((uint16_t)(x[i] & 0xffffu), DT);
+      v[0][2 * i + 1] = to_f32_16((uint16_t)(x[i] >> 16), DT);
     }
-    // stages 1, 2, 4, ...: (u, v) -> (u + v, u - v) in fp32 (compressor.py:34-39)
 #pragma unroll
     for (int lh = 0; lh < 3; ++lh) {
       if (lh < log_had) {
@@ -288,6 +261,94 @@ __global__ void __launch_bounds__(kMidPrepThreads) mid_prep_kernel(const uint16_
     if (log_had > 6) prep_fly<8>(v, side(8), lane);
     if (log_had > 7) prep_fly<16>(v, side(16), lane);
     if (log_had > 8) prep_fly<32>(v, side(32), lane);
+    return sgn;
+  };
+  uint32_t mb = 0;  // fp32 bits of the largest magnitude: an infinity above every number, NaN above all
+  if (log_had > 0) {
+    // A maximum needs the block's outputs in no order and with no sign: lanes meet at distances
+    // 1, 2, 7, 8 (all single DPP operands; a lane's sides are then bits 0 ^ 2, 1 ^ 2, 2, 3), and the
+    // stage inside a dword comes last, max(|u + v|, |u - v|) = |u| + |v|.  What the order moves the
+    // maximum by (2^-22) can turn the exponent at its edge only, inside fp16's spare octave.
+    const float s1 = ((lane ^ (lane >> 2)) & 1) ? -1.0f : 1.0f, s2 = ((lane ^ (lane >> 1)) & 2) ? -1.0f : 1.0f;
+    const float s4 = (lane & 4) ? -1.0f : 1.0f, s8 = (lane & 8) ? -1.0f : 1.0f;
+    auto block_max = [&](const mu4_t& x) __attribute__((always_inline)) {
+      float v[1][8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[0][2 * i] = to_f32_16((uint16_t)(x[i] & 0xffffu), DT);
+        v[0][2 * i + 1] = to_f32_16((uint16_t)(x[i] >> 16), DT);
+      }
+#pragma unroll
+      for (int lh = 1; lh < 3; ++lh)
+        if (lh < log_had)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if ((e & (1 << lh)) == 0) {
+              const float x0 = v[0][e], x1 = v[0][e | (1 << lh)];
+              v[0][e] = x0 + x1;
+              v[0][e | (1 << lh)] = x0 - x1;
+            }
+      if (log_had > 3) prep_fly<1>(v, s1, lane);
+      if (log_had > 4) prep_fly<2>(v, s2, lane);
+      if (log_had > 5) prep_fly<7>(v, s4, lane);
+      if (log_had > 6) prep_fly<8>(v, s8, lane);
+      if (log_had > 7) prep_fly<16>(v, (lane & 16) ? -1.0f : 1.0f, lane);
+      if (log_had > 8) prep_fly<32>(v, (lane & 32) ? -1.0f : 1.0f, lane);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        mb = max(mb, __builtin_bit_cast(uint32_t, fabsf(v[0][2 * i]) + fabsf(v[0][2 * i + 1])) & 0x7fffffffu);
+    };
+    constexpr int B = 8;  // loads in flight; a lane past the end takes its piece of the first block again
+    const int e0 = 8 * lane, back = e0 & ((1 << log_had) - 1);
+    for (int b = 0; b < k; b += B * kMidPrepSeg) {
+      mu4_t f[B];
+#pragma unroll
+      for (int j = 0; j < B; ++j) f[j] = load8(b + kMidPrepSeg * j + e0 < k ? b + kMidPrepSeg * j + e0 : back);
+#pragma unroll
+      for (int j = 0; j < B; ++j) {
+        if (b + kMidPrepSeg * j >= k) break;
+        block_max(f[j]);
+      }
+    }
+  } else {
+    mus2_t mx = {0, 0};
+    for (int e = 8 * lane; e < k; e += 16 * kMidPrepSeg) {  // sixteen loads in flight
+      mu4_t f[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) f[j] = load8(e + kMidPrepSeg * j < k ? e + kMidPrepSeg * j : e);
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          mx = __builtin_elementwise_max(mx, __builtin_bit_cast(mus2_t, f[j][i] & 0x7fff7fffu));
+    }
+    mb = max(__builtin_bit_cast(uint32_t, to_f32_16(mx[0], DT)), __builtin_bit_cast(uint32_t, to_f32_16(mx[1], DT)));
+  }
+  auto partner = [&](float other) { mb = max(mb, __builtin_bit_cast(uint32_t, other)); };
+  partner(lane_xor<32>(__builtin_bit_cast(float, mb), lane));
+  partner(lane_xor<16>(__builtin_bit_cast(float, mb), lane));
+  partner(lane_xor<8>(__builtin_bit_cast(float, mb), lane));
+  partner(lane_xor<4>(__builtin_bit_cast(float, mb), lane));
+  partner(lane_xor<2>(__builtin_bit_cast(float, mb), lane));
+  partner(lane_xor<1>(__builtin_bit_cast(float, mb), lane));
+  const uint32_t bits = log_had > 0 ? __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, mb) / div) : mb;
+  const int eb = (int)(bits >> 23);
+  const int E = eb == 0 ? -126 : eb - 127;
+  int F = bits == 0 || mb > 0x7f800000u ? 0 : 14 - E;  // (NaN takes the whole row at any scale)
+  F = F < -126 ? -126 : (F > 126 ? 126 : F);
+  if (s0 == 0 && lane == 0 && r0 + wv < m) fexp[r0 + wv] = F;
+  const float f2 = __builtin_bit_cast(float, (uint32_t)(F + 127) << 23);
+  // unit of this lane in its 32-run (lane & 3 = q holds elements 8 q .. 8 q + 7): plain order,
+  // elements 8 q ..; Marlin order, the pairs (k, k + 16) for k = 4 d .. 4 d + 3, which the
+  // lanes q and q ^ 2 build from each other's halves (d = 0, 2, 1, 3 for q = 0, 1, 2, 3)
+  const int q = lane & 3;
+  const int d = marlin ? ((q & 1) << 1) | (q >> 1) : q;
+  const int nc = k >> 6, t = r0 >> 5, rl = r0 & 31;
+  for (int sg = s0; sg < min(s0 + segs, nseg); ++sg) {
+    const int k0 = sg * kMidPrepSeg;
+    const mu4_t x = load8(k0 + 8 * lane < k ? k0 + 8 * lane : 0);  // k is a multiple of 64
+    float v[1][8];
+    const float sgn = rotate(x, v);
     const float f = sgn * (log_had > 0 ? f2 / div : f2);
     mu4_t w;
     if (marlin) {
@@ -791,11 +852,13 @@ int mid_launch(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m
   const int segs = std::max(1, (rg * nseg + kMidPrepWgs - 1) / kMidPrepWgs);
   const int xblocks = rg * ((nseg + segs - 1) / segs);
   const int sblocks = g.nt * (kMidBN / kMidEntryRows) * (int)((w->k + 2047) / 2048);
-  const void* prep = vec ? (const void*)mid_prep_kernel<true> : (const void*)mid_prep_kernel<false>;
+  const void* prep = act_dtype == SPECTRA_BF16
+                         ? (vec ? (const void*)mid_prep_kernel<true, SPECTRA_BF16> : (const void*)mid_prep_kernel<false, SPECTRA_BF16>)
+                         : (vec ? (const void*)mid_prep_kernel<true, SPECTRA_F16> : (const void*)mid_prep_kernel<false, SPECTRA_F16>);
   const int mi = (int)m, marlin = w->marlin_layout ? 1 : 0;
   uint16_t *frag = (uint16_t*)(ws + l.frag), *xk = has_o ? (uint16_t*)(ws + l.xk) : nullptr;
   int32_t* fexp = (int32_t*)(ws + l.fexp);
-  void* pargs[] = {(void*)&a, (void*)&lda, (void*)&act_dtype, (void*)&mi, (void*)&p.k, (void*)&log_had, (void*)&div,
+  void* pargs[] = {(void*)&a, (void*)&lda, (void*)&mi, (void*)&p.k, (void*)&log_had, (void*)&div,
                    (void*)&marlin, (void*)&frag, (void*)&xk, (void*)&p.mp, (void*)&fexp, (void*)&sblocks, (void*)&segs, (void*)&en};
   SPECTRA_HIP_CHECK(hipLaunchKernel(prep, dim3((unsigned)(xblocks + sblocks)), dim3(kMidPrepThreads), pargs, 0, s));
   SPECTRA_HIP_CHECK(hipGetLastError());

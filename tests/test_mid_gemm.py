@@ -118,3 +118,22 @@ def test_mid_strides_alignment_and_workspace(hip):
         assert st == 0
         _check(out[:, :n], x, _dense(q), 128, None, "float16")
         assert bool((out[:, n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("had", [0, 128, 512])
+def test_mid_row_scale(hip, had):
+    """Small activations beside one huge one, whose block meets only zero weights: the row scale is
+    that of the rotated row (60000 / sqrt(b)), so the others, 2^-22 to 2^-24 of it, keep fp16's 11
+    bits.  Bound as above."""
+    m, n, k = 40, 256, 1024
+    g = torch.Generator(device="cuda").manual_seed(had)
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    w[:, :512] = 0
+    q = C.quantize_nf4(w.half(), 64, 0, None, True)
+    x = (torch.rand(m, k, generator=g, device="cuda") + 0.5) * (2e-4 if had else 8e-3)
+    x[:, :512] = 0
+    x[:, 3] = 60000.0
+    x = x.half()
+    y = K.batched_w4a16_gemm(x, q.packed, q.absmax, None, None, None, True, codebook="nf4", group_size=64,
+                             hadamard_block=had)
+    _check(y, x, _dense(q), had, None, "float16")
