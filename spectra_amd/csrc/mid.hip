@@ -52,7 +52,7 @@ struct MidParams {
   int64_t ldo;
   float* part;  // fp32 partials [ksplit][mp / 32][np / 32][32 x 32 in accumulator order]
   int m, n, k, mp, np;
-  int n_out, has_o, bias_dt, act_dt;
+  int n_out, has_o, asym, marlin, bias_dt, act_dt;
   int ksplit, chunks;  // K splits (blockIdx.z) and 64-k chunks per split
 };
 
@@ -623,6 +623,43 @@ __global__ void __launch_bounds__(kMidThreads) mid_kernel(const MidParams p) {
   }
 }
 
+// Rows with an infinity have the scale exponent kMidInfF, which no finite row reaches.  Where the
+// weight has outliers such a row's products are summed here, value x inf in place of code x inf (a
+// code of 0 would make it NaN); what its finite activations add does not show beside an infinity.
+constexpr int kMidInfF = 14 - 128;
+__device__ __forceinline__ float mid_inf_row(const MidParams& p, int row, int col, float y0) {
+  const int e0 = p.rowptr ? p.rowptr[col] : col * p.n_out, e1 = p.rowptr ? p.rowptr[col + 1] : e0 + p.n_out;
+  const int NC = p.k >> 6;
+  float y = 0.0f;
+  bool any = false;
+#pragma unroll 16
+  for (int k = 0; k < p.k; ++k) {
+    const uint16_t x = p.xk[(int64_t)k * p.mp + row];
+    if ((x & 0x7c00) != 0x7c00) continue;
+    any = true;
+    int64_t bj;
+    int hb;
+    k_to_nibble(k, p.marlin, &bj, &hb);
+    const int code = (p.packed[(int64_t)col * p.ldp + bj] >> (4 * hb)) & 15;
+    const int64_t si = ((int64_t)(col >> 5) * NC + (k >> 6)) * 64 + (k & 32) + (col & 31);
+    float w;
+    if (p.asym) {
+      const uint32_t sz = ((const uint32_t*)p.sfrag)[si];
+      w = ((float)(1024 + code) + h2f((uint16_t)(sz >> 16))) * h2f((uint16_t)sz);
+    } else {
+      w = h2f(nf4_f16_bits(code)) * h2f(((const uint16_t*)p.sfrag)[si]);
+    }
+    w = h2f(f2h(w));
+    float v = w;
+    for (int e = e0; e < e1; ++e) {
+      const uint2 m = p.meta[e];
+      if ((int)m.x == k) v = w + __builtin_bit_cast(float, m.y);
+    }
+    y = __builtin_fmaf(v, h2f(x), y);
+  }
+  return any ? y : y0;
+}
+
 // out = act((sum over splits of the partials + outliers) 2^-F + bias), 32 columns x RB row tiles
 // per workgroup, splits summed in order.  Groups of RB * 8 lanes (four rows a lane) own a
 // column's entries, twelve reads of the k-major activations in flight; the 512 threads are
@@ -701,7 +738,8 @@ __global__ void __launch_bounds__(kMidRedThreads) mid_reduce_kernel(const MidPar
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int F = p.fexp[min(m0 + rl + e, p.m - 1)];
+      const int row = min(m0 + rl + e, p.m - 1), F = p.fexp[row];
+      if (p.has_o && F == kMidInfF && col < p.n) y[e] = mid_inf_row(p, row, col, y[e]);
       ot[rl + e][tid & 31] = from_f32_16(y[e] * __builtin_bit_cast(float, (uint32_t)(127 - F) << 23) + bv, p.act_dt);
     }
   }
@@ -831,6 +869,7 @@ int mid_launch(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m
   p.part = (float*)(ws + l.part);
   p.m = (int)m; p.n = (int)w->n; p.k = (int)w->k; p.mp = g.mp; p.np = g.nt * kMidBN;
   p.n_out = w->num_outliers; p.has_o = has_o;
+  p.asym = w->format == SPECTRA_FMT_ASYM_G32; p.marlin = w->marlin_layout ? 1 : 0;
   p.bias_dt = w->bias_dtype; p.act_dt = act_dtype;
   p.ksplit = g.ksplit; p.chunks = g.chunks;
   MidSide en;

@@ -137,3 +137,37 @@ def test_mid_row_scale(hip, had):
     y = K.batched_w4a16_gemm(x, q.packed, q.absmax, None, None, None, True, codebook="nf4", group_size=64,
                              hadamard_block=had)
     _check(y, x, _dense(q), had, None, "float16")
+
+
+@pytest.mark.parametrize("fmt", ["nf4", "asym"])
+def test_mid_infinite_activations(hip, fmt):
+    """An infinite activation at an outlier gives value x inf, not NaN (the code under an outlier is
+    0); one elsewhere meets codes of 0 too and gives NaN there, as the product of W_eff does."""
+    m, n, k = 40, 256, 1024
+    g = torch.Generator(device="cuda").manual_seed(3)
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    if fmt == "nf4":
+        mask = torch.rand(n, k, generator=g, device="cuda") < 0.01
+        mask[:, 5] = True
+        mask[:, 700] = True
+        q = C.quantize_nf4(torch.where(mask, w * 10, w).half(), 64, 0, mask, True)
+        args = (q.packed, q.absmax, None, q.col, q.val, True)
+        kw = dict(codebook="nf4", group_size=64, outlier_rowptr=q.rowptr)
+    else:
+        idx = torch.tensor([5, 300, 700], device="cuda")
+        packed, scales, pz = C.quantize_group32(w, 32, idx)
+        args = (packed, scales, C.unpack_zeros(pz, k).contiguous(), idx, (w[:, idx] * 10).half().contiguous(), True)
+        kw = {}
+    x = torch.randn(m, k, generator=g, device="cuda").half()
+    inf = float("inf")
+    x[3, 5], x[4, 5], x[4, 700], x[38, 700], x[39, 6], x[20, 9] = inf, -inf, inf, -inf, inf, float("nan")
+    y = K.batched_w4a16_gemm(x, *args, **kw).cpu()
+    dkw = {a: b for a, b in kw.items() if a != "group_size"}
+    weff = K.w4_dequant(*args[:3], out_dtype=torch.float32, marlin_layout=True, outlier_idx=args[3],
+                        outlier_w=args[4], **dkw).cpu()
+    ref = (x.cpu().double()[:, None] * weff.double()[None]).sum(-1)
+    special = ~ref.isfinite()
+    assert special[[3, 4, 20, 38, 39]].all() and ref[3].isinf().all() and ref[38].isinf().all()
+    assert torch.equal(y.double()[special].nan_to_num(7.0, 8.0, 9.0), ref[special].nan_to_num(7.0, 8.0, 9.0))
+    fin = ~special
+    assert ((y.double() - ref)[fin].norm() / ref[fin].norm()).item() <= 1e-3
