@@ -192,13 +192,14 @@ __device__ __forceinline__ void mid_entries(const MidSide& en, int k, int marlin
 }
 
 // Workgroups [0, sblocks): block scales and outlier entries; the others: 8 rows (one per wave) x
-// segs 512-k segments (lane l: elements 8 l .. 8 l + 7 of each).  The row scale, max |x_rot| 2^F in
-// [2^14, 2^15), is every workgroup's own pass over the whole rotated row: with a bound from the raw row
-// (sqrt(b) max |x|) one large activation cost the small ones up to 4.5 of fp16's octaves.  Without a
-// rotation magnitudes are compared as 15-bit integers, two to an instruction (an infinity or a NaN is
-// the largest and takes its own row with it, as any product would).  FWHT stages 1, 2, 4 run in
-// registers, 8 .. 256 across lanes.  Fragments leave through LDS in whole 128-byte lines (8 rows x
-// 16 bytes); the k-major copy in 16-byte pieces.
+// segs 512-k segments (lane l: elements 8 l .. 8 l + 7 of each).  The row scale is every workgroup's
+// own from the whole row.  max |x_rot| 2^F lies in [2^14, 2^15), or, where the raw row is even (every
+// nonzero piece of 8 reaches 2^-10 of its maximum), the bound sqrt(b) max |x| does: a block's energy is
+// then at least 2^-5 per element, 2^20 above what fp16 can drop there.  A bound alone cost a row
+// with one large activation up to 4.5 octaves of its small blocks' range; the maximum alone, a
+// transform of the whole row in every workgroup, QKV 0.8 us at 48 rows and down 3.  FWHT
+// stages 1, 2, 4 run in registers, 8 .. 256 across lanes.  Fragments leave through LDS in whole
+// 128-byte lines (8 rows x 16 bytes); the k-major copy in 16-byte pieces.
 template <bool VEC, int DT>
 __global__ void __launch_bounds__(kMidPrepThreads) mid_prep_kernel(const uint16_t* __restrict__ a, int64_t lda, int m,
                                                                     int k, int log_had, float div, int marlin,
@@ -263,75 +264,94 @@ __global__ void __launch_bounds__(kMidPrepThreads) mid_prep_kernel(const uint16_
     if (log_had > 8) prep_fly<32>(v, side(32), lane);
     return sgn;
   };
-  uint32_t mb = 0;  // fp32 bits of the largest magnitude: an infinity above every number, NaN above all
-  if (log_had > 0) {
-    // A maximum needs the block's outputs in no order and with no sign: lanes meet at distances
-    // 1, 2, 7, 8 (all single DPP operands; a lane's sides are then bits 0 ^ 2, 1 ^ 2, 2, 3), and the
-    // stage inside a dword comes last, max(|u + v|, |u - v|) = |u| + |v|.  What the order moves the
-    // maximum by (2^-22) can turn the exponent at its edge only, inside fp16's spare octave.
-    const float s1 = ((lane ^ (lane >> 2)) & 1) ? -1.0f : 1.0f, s2 = ((lane ^ (lane >> 1)) & 2) ? -1.0f : 1.0f;
-    const float s4 = (lane & 4) ? -1.0f : 1.0f, s8 = (lane & 8) ? -1.0f : 1.0f;
-    auto block_max = [&](const mu4_t& x) __attribute__((always_inline)) {
-      float v[1][8];
+  // the raw row: its largest magnitude, and the smallest one that a lane's nonzero piece of 8 reaches,
+  // as 15-bit integers, two to an instruction (an infinity or a NaN is the largest)
+  mus2_t mx = {0, 0};
+  uint32_t mn = 0x7fff;  // less 1
+  for (int e = 8 * lane; e < k; e += 16 * kMidPrepSeg) {  // sixteen loads in flight (past the end: the first again)
+    mu4_t f[16];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[0][2 * i] = to_f32_16((uint16_t)(x[i] & 0xffffu), DT);
-        v[0][2 * i + 1] = to_f32_16((uint16_t)(x[i] >> 16), DT);
-      }
+    for (int j = 0; j < 16; ++j) f[j] = load8(e + kMidPrepSeg * j < k ? e + kMidPrepSeg * j : e);
 #pragma unroll
-      for (int lh = 1; lh < 3; ++lh)
-        if (lh < log_had)
+    for (int j = 0; j < 16; ++j) {
+      mus2_t c = {0, 0};
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if ((e & (1 << lh)) == 0) {
-              const float x0 = v[0][e], x1 = v[0][e | (1 << lh)];
-              v[0][e] = x0 + x1;
-              v[0][e | (1 << lh)] = x0 - x1;
-            }
-      if (log_had > 3) prep_fly<1>(v, s1, lane);
-      if (log_had > 4) prep_fly<2>(v, s2, lane);
-      if (log_had > 5) prep_fly<7>(v, s4, lane);
-      if (log_had > 6) prep_fly<8>(v, s8, lane);
-      if (log_had > 7) prep_fly<16>(v, (lane & 16) ? -1.0f : 1.0f, lane);
-      if (log_had > 8) prep_fly<32>(v, (lane & 32) ? -1.0f : 1.0f, lane);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        mb = max(mb, __builtin_bit_cast(uint32_t, fabsf(v[0][2 * i]) + fabsf(v[0][2 * i + 1])) & 0x7fffffffu);
-    };
-    constexpr int B = 8;  // loads in flight; a lane past the end takes its piece of the first block again
-    const int e0 = 8 * lane, back = e0 & ((1 << log_had) - 1);
-    for (int b = 0; b < k; b += B * kMidPrepSeg) {
-      mu4_t f[B];
-#pragma unroll
-      for (int j = 0; j < B; ++j) f[j] = load8(b + kMidPrepSeg * j + e0 < k ? b + kMidPrepSeg * j + e0 : back);
-#pragma unroll
-      for (int j = 0; j < B; ++j) {
-        if (b + kMidPrepSeg * j >= k) break;
-        block_max(f[j]);
-      }
+      for (int i = 0; i < 4; ++i) c = __builtin_elementwise_max(c, __builtin_bit_cast(mus2_t, f[j][i] & 0x7fff7fffu));
+      mx = __builtin_elementwise_max(mx, c);
+      mn = min(mn, (uint32_t)max(c[0], c[1]) - 1u);
     }
-  } else {
-    mus2_t mx = {0, 0};
-    for (int e = 8 * lane; e < k; e += 16 * kMidPrepSeg) {  // sixteen loads in flight
-      mu4_t f[16];
+  }
+  // fp32 bits: an infinity above every number, NaN above all
+  uint32_t mb = max(__builtin_bit_cast(uint32_t, to_f32_16(mx[0], DT)), __builtin_bit_cast(uint32_t, to_f32_16(mx[1], DT)));
+  auto wave_max_bits = [&](uint32_t v) __attribute__((always_inline)) {
+    auto with = [&](float o) { v = max(v, __builtin_bit_cast(uint32_t, o)); };
+    with(lane_xor<32>(__builtin_bit_cast(float, v), lane));
+    with(lane_xor<16>(__builtin_bit_cast(float, v), lane));
+    with(lane_xor<8>(__builtin_bit_cast(float, v), lane));
+    with(lane_xor<4>(__builtin_bit_cast(float, v), lane));
+    with(lane_xor<2>(__builtin_bit_cast(float, v), lane));
+    with(lane_xor<1>(__builtin_bit_cast(float, v), lane));
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+  };
+  mb = wave_max_bits(mb);
+  uint32_t bits = mb;
+  if (log_had > 0) {
+    const float raw = __builtin_bit_cast(float, mb), bound = raw * div * 1.0009765625f;
+    const uint32_t least = 0x8000u - wave_max_bits(0x7fffu - mn);  // (0x8000: no nonzero piece)
+    const bool even = log_had >= 3 && bound < __builtin_inff() &&
+                      (least == 0x8000u || to_f32_16((uint16_t)least, DT) >= raw * 0x1p-10f);
+    bits = __builtin_bit_cast(uint32_t, bound);
+    if (!even) {
+      mb = 0;
+      // A maximum needs the block's outputs in no order and with no sign: lanes meet at distances
+      // 1, 2, 7, 8 (all single DPP operands; a lane's sides are then bits 0 ^ 2, 1 ^ 2, 2, 3), and the
+      // stage inside a dword comes last, max(|u + v|, |u - v|) = |u| + |v|.  What the order moves the
+      // maximum by (2^-22) can turn the exponent at its edge only, inside fp16's spare octave.
+      const float s1 = ((lane ^ (lane >> 2)) & 1) ? -1.0f : 1.0f, s2 = ((lane ^ (lane >> 1)) & 2) ? -1.0f : 1.0f;
+      const float s4 = (lane & 4) ? -1.0f : 1.0f, s8 = (lane & 8) ? -1.0f : 1.0f;
+      auto block_max = [&](const mu4_t& x) __attribute__((always_inline)) {
+        float v[1][8];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) f[j] = load8(e + kMidPrepSeg * j < k ? e + kMidPrepSeg * j : e);
+        for (int i = 0; i < 4; ++i) {
+          v[0][2 * i] = to_f32_16((uint16_t)(x[i] & 0xffffu), DT);
+          v[0][2 * i + 1] = to_f32_16((uint16_t)(x[i] >> 16), DT);
+        }
 #pragma unroll
-      for (int j = 0; j < 16; ++j)
+        for (int lh = 1; lh < 3; ++lh)
+          if (lh < log_had)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if ((e & (1 << lh)) == 0) {
+                const float x0 = v[0][e], x1 = v[0][e | (1 << lh)];
+                v[0][e] = x0 + x1;
+                v[0][e | (1 << lh)] = x0 - x1;
+              }
+        if (log_had > 3) prep_fly<1>(v, s1, lane);
+        if (log_had > 4) prep_fly<2>(v, s2, lane);
+        if (log_had > 5) prep_fly<7>(v, s4, lane);
+        if (log_had > 6) prep_fly<8>(v, s8, lane);
+        if (log_had > 7) prep_fly<16>(v, (lane & 16) ? -1.0f : 1.0f, lane);
+        if (log_had > 8) prep_fly<32>(v, (lane & 32) ? -1.0f : 1.0f, lane);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          mx = __builtin_elementwise_max(mx, __builtin_bit_cast(mus2_t, f[j][i] & 0x7fff7fffu));
+          mb = max(mb, __builtin_bit_cast(uint32_t, fabsf(v[0][2 * i]) + fabsf(v[0][2 * i + 1])) & 0x7fffffffu);
+      };
+      constexpr int B = 8;  // loads in flight; a lane past the end takes its piece of the first block again
+      const int e0 = 8 * lane, back = e0 & ((1 << log_had) - 1);
+      for (int b = 0; b < k; b += B * kMidPrepSeg) {
+        mu4_t f[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j) f[j] = load8(b + kMidPrepSeg * j + e0 < k ? b + kMidPrepSeg * j + e0 : back);
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+          if (b + kMidPrepSeg * j >= k) break;
+          block_max(f[j]);
+        }
+      }
+      mb = wave_max_bits(mb);
+      bits = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, mb) / div);
     }
-    mb = max(__builtin_bit_cast(uint32_t, to_f32_16(mx[0], DT)), __builtin_bit_cast(uint32_t, to_f32_16(mx[1], DT)));
   }
-  auto partner = [&](float other) { mb = max(mb, __builtin_bit_cast(uint32_t, other)); };
-  partner(lane_xor<32>(__builtin_bit_cast(float, mb), lane));
-  partner(lane_xor<16>(__builtin_bit_cast(float, mb), lane));
-  partner(lane_xor<8>(__builtin_bit_cast(float, mb), lane));
-  partner(lane_xor<4>(__builtin_bit_cast(float, mb), lane));
-  partner(lane_xor<2>(__builtin_bit_cast(float, mb), lane));
-  partner(lane_xor<1>(__builtin_bit_cast(float, mb), lane));
-  const uint32_t bits = log_had > 0 ? __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, mb) / div) : mb;
   const int eb = (int)(bits >> 23);
   const int E = eb == 0 ? -126 : eb - 127;
   int F = bits == 0 || mb > 0x7f800000u ? 0 : 14 - E;  // (NaN takes the whole row at any scale)
