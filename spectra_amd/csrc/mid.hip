@@ -52,7 +52,7 @@ struct MidParams {
   int64_t ldo;
   float* part;  // fp32 partials [ksplit][mp / 32][np / 32][32 x 32 in accumulator order]
   int m, n, k, mp, np;
-  int n_out, has_o, asym, marlin, bias_dt, act_dt;
+  int n_out, has_o, cap, asym, marlin, bias_dt, act_dt;  // cap: entries of a row its own lanes add
   int ksplit, chunks;  // K splits (blockIdx.z) and 64-k chunks per split
 };
 
@@ -683,13 +683,20 @@ __device__ __forceinline__ float mid_inf_row(const MidParams& p, int row, int co
 // out = act((sum over splits of the partials + outliers) 2^-F + bias), 32 columns x RB row tiles
 // per workgroup, splits summed in order.  Groups of RB * 8 lanes (four rows a lane) own a
 // column's entries, twelve reads of the k-major activations in flight; the 512 threads are
-// 64 / RB such groups, CG of them (64 / RB / 32) sharing a column.
+// 64 / RB such groups, CG of them (64 / RB / 32) sharing a column.  A row much longer than the others
+// would run on alone: past p.cap entries (twice the average, at least 64) all groups share it.  48 rows
+// of 3072 x 8192, 0.5% outliers: 37.7 us, one dense row 623 without that and 71 with it (the 256-row
+// tiles: 74).
 constexpr int kMidRedThreads = 512, kMidMaxSplit = 16;
 template <int RB>
 __global__ void __launch_bounds__(kMidRedThreads) mid_reduce_kernel(const MidParams p) {
   constexpr int LP = 8 * RB, CG = kMidRedThreads / LP / 32, RS = 32 * RB + 4;
   __shared__ __align__(16) float cor[CG][32][RS];
   __shared__ __align__(16) uint16_t ot[32 * RB][32 + 8];
+  constexpr int NG = kMidRedThreads / LP;
+  __shared__ __align__(16) float tail[NG][RS];  // long rows: the groups' sums
+  __shared__ int2 rows[32];
+  __shared__ int longer[kMidRedThreads / 64];
   const int tid = threadIdx.x;
   const int nb = blockIdx.y, n0 = 32 * nb, tb = blockIdx.x * RB, m0 = 32 * tb;
   const int NB = p.np >> 5, MB = p.mp >> 5;
@@ -701,36 +708,63 @@ __global__ void __launch_bounds__(kMidRedThreads) mid_reduce_kernel(const MidPar
 #pragma unroll
   for (int v = 0; v < 8; ++v) pb[v] = *(const float4*)(src + min(v, p.ksplit - 1) * zs);
   if (p.has_o) {
-    const int grp = tid / LP, lr = tid % LP, c = min(n0 + (grp & 31), p.n - 1), cg = grp >> 5;
-    const int e0 = p.rowptr ? p.rowptr[c] : c * p.n_out, e1 = p.rowptr ? p.rowptr[c + 1] : e0 + p.n_out;
+    const int grp = tid / LP, lr = tid % LP, cg = grp >> 5;
     const uint16_t* xsrc = p.xk + m0 + 4 * lr;
-    float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    constexpr int U = 12;
-    uint2 md[U];  // the next turn's entries are read while this turn's activations are on the way
-    if (e0 + cg < e1)
+    // entries e, e + step, ... of [.., e1) into o
+    auto gather = [&](int e, const int e1, const int step, float (&o)[4]) __attribute__((always_inline)) {
+      constexpr int U = 12;
+      uint2 md[U];  // the next turn's entries are read while this turn's activations are on the way
+      if (e < e1)
 #pragma unroll
-      for (int v = 0; v < U; ++v) md[v] = p.meta[min(e0 + cg + v * CG, e1 - 1)];
-    for (int e = e0 + cg; e < e1; e += U * CG) {
-      uint2 x[U];
-      float d[U];
+        for (int v = 0; v < U; ++v) md[v] = p.meta[min(e + v * step, e1 - 1)];
+      for (; e < e1; e += U * step) {
+        uint2 x[U];
+        float d[U];
 #pragma unroll
-      for (int v = 0; v < U; ++v) {
-        x[v] = *(const uint2*)(xsrc + (int64_t)md[v].x * p.mp);
-        d[v] = e + v * CG < e1 ? __builtin_bit_cast(float, md[v].y) : 0.0f;
-      }
-#pragma unroll
-      for (int v = 0; v < U; ++v) md[v] = p.meta[min(e + (U + v) * CG, e1 - 1)];
-#pragma unroll
-      for (int v = 0; v < U; ++v)
-        if (e + v * CG < e1) {
-          o[0] = __builtin_fmaf(d[v], h2f((uint16_t)x[v].x), o[0]);
-          o[1] = __builtin_fmaf(d[v], h2f((uint16_t)(x[v].x >> 16)), o[1]);
-          o[2] = __builtin_fmaf(d[v], h2f((uint16_t)x[v].y), o[2]);
-          o[3] = __builtin_fmaf(d[v], h2f((uint16_t)(x[v].y >> 16)), o[3]);
+        for (int v = 0; v < U; ++v) {
+          x[v] = *(const uint2*)(xsrc + (int64_t)md[v].x * p.mp);
+          d[v] = e + v * step < e1 ? __builtin_bit_cast(float, md[v].y) : 0.0f;
         }
-    }
+#pragma unroll
+        for (int v = 0; v < U; ++v) md[v] = p.meta[min(e + (U + v) * step, e1 - 1)];
+#pragma unroll
+        for (int v = 0; v < U; ++v)
+          if (e + v * step < e1) {
+            o[0] = __builtin_fmaf(d[v], h2f((uint16_t)x[v].x), o[0]);
+            o[1] = __builtin_fmaf(d[v], h2f((uint16_t)(x[v].x >> 16)), o[1]);
+            o[2] = __builtin_fmaf(d[v], h2f((uint16_t)x[v].y), o[2]);
+            o[3] = __builtin_fmaf(d[v], h2f((uint16_t)(x[v].y >> 16)), o[3]);
+          }
+      }
+    };
+    const int c = min(n0 + (grp & 31), p.n - 1);
+    const int e0 = p.rowptr ? p.rowptr[c] : c * p.n_out, e1 = p.rowptr ? p.rowptr[c + 1] : e0 + p.n_out;
+    if (grp < 32 && lr == 0) rows[grp] = make_int2(e0, e1);
+    float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    gather(e0 + cg, e0 + min(e1 - e0, p.cap), CG, o);
+    const bool any = __builtin_amdgcn_ballot_w64(e1 - e0 > p.cap) != 0;
+    if ((tid & 63) == 0) longer[tid >> 6] = any;
     *(float4*)&cor[cg][grp & 31][4 * lr] = make_float4(o[0], o[1], o[2], o[3]);
     __syncthreads();
+    int more = 0;
+#pragma unroll
+    for (int w = 0; w < kMidRedThreads / 64; ++w) more |= longer[w];
+    if (more) {
+      for (int j = 0; j < min(32, p.n - n0); ++j) {
+        const int2 r = rows[j];
+        if (r.y - r.x <= p.cap) continue;  // (uniform)
+        float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        gather(r.x + p.cap + grp, r.y, NG, t);
+        *(float4*)&tail[grp][4 * lr] = make_float4(t[0], t[1], t[2], t[3]);
+        __syncthreads();
+        if (tid < 32 * RB) {
+          float v = cor[0][j][tid];
+          for (int g = 0; g < NG; ++g) v += tail[g][tid];
+          cor[0][j][tid] = v;
+        }
+        __syncthreads();
+      }
+    }
   }
   float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   for (int z0 = 0;;) {
@@ -889,6 +923,7 @@ int mid_launch(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m
   p.part = (float*)(ws + l.part);
   p.m = (int)m; p.n = (int)w->n; p.k = (int)w->k; p.mp = g.mp; p.np = g.nt * kMidBN;
   p.n_out = w->num_outliers; p.has_o = has_o;
+  p.cap = (int)std::max<int64_t>(64, 2 * mid_entries_count(w) / w->n);
   p.asym = w->format == SPECTRA_FMT_ASYM_G32; p.marlin = w->marlin_layout ? 1 : 0;
   p.bias_dt = w->bias_dtype; p.act_dt = act_dtype;
   p.ksplit = g.ksplit; p.chunks = g.chunks;

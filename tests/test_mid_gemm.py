@@ -171,3 +171,39 @@ def test_mid_infinite_activations(hip, fmt):
     assert torch.equal(y.double()[special].nan_to_num(7.0, 8.0, 9.0), ref[special].nan_to_num(7.0, 8.0, 9.0))
     fin = ~special
     assert ((y.double() - ref)[fin].norm() / ref[fin].norm()).item() <= 1e-3
+
+
+def test_mid_long_outlier_rows(hip):
+    """Rows far longer than the others (every column, every second one, one tile's worth more than the
+    lanes of a row add by themselves): right, and shared among the workgroup's lanes: one row of 8192
+    entries took 16 times a call with short rows only when its own lanes added it, 1.9 times now."""
+    n, k = 3072, 8192
+    g = torch.Generator(device="cuda").manual_seed(9)
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    mask = torch.rand(n, k, generator=g, device="cuda") < 0.005
+    times = []
+    for dense in (False, True):
+        if dense:
+            mask[7], mask[40, ::2], mask[41, :200], mask[n - 1, 5:] = True, True, True, True
+        q = C.quantize_nf4(torch.where(mask, w * 10, w).half(), 64, 0, mask, True)
+        for m in (20, 48):
+            x = torch.randn(m, k, generator=g, device="cuda").half()
+
+            def call():
+                return K.batched_w4a16_gemm(x, q.packed, q.absmax, None, q.col, q.val, True, codebook="nf4",
+                                            group_size=64, outlier_rowptr=q.rowptr)
+            y = call()
+            _check(y, x, _dense(q), 0, None, "float16")
+            assert torch.equal(call(), y)
+        call()
+        best = 1e9
+        for _ in range(10):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                call()
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        times.append(best)
+    assert times[1] <= 6 * times[0], times
