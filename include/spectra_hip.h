@@ -147,7 +147,8 @@ int spectra_w4a16_gemv_fused(const spectra_qweight_t* w, const void* x, int64_t 
  * Batched / prefill GEMM family (any M >= 1, MFMA):
  *   out = FWHT_hb(a) . W_eff^T + bias,   fp32 accumulation.
  * a: act_dtype [m, K] row stride lda; out: act_dtype [m, N] row stride ldo.
- * 2 <= m <= 16: small-batch stream; otherwise the hand-written GEMM (fp16 operands); from
+ * 2 <= m <= 16: small-batch stream; otherwise the hand-written GEMMs (fp16 operands: a mid-size
+ * family and 256-row tiles); from
  * m >= 512, when the workspace holds it, W_eff dequantized into the workspace in act_dtype
  * and one hipBLASLt GEMM on it (the reference kernel's operand rounding).
  * workspace: device scratch of spectra_w4a16_gemm_workspace() bytes, which serves every
@@ -156,6 +157,9 @@ int spectra_w4a16_gemv_fused(const spectra_qweight_t* w, const void* x, int64_t 
  * the size is 0.  Replaces kernels.py:333-389.
  */
 size_t spectra_w4a16_gemm_workspace(const spectra_qweight_t* w, int64_t m, int32_t act_dtype);
+/* 1 when spectra_w4a16_gemm runs m rows with that much workspace on the mid-size family (some of
+ * 17 <= m < 512, by the weight's shape and outlier density), 0 when on another; launches nothing. */
+int spectra_w4a16_gemm_mid(const spectra_qweight_t* w, int64_t m, size_t workspace_bytes);
 int spectra_w4a16_gemm(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m,
                        int32_t act_dtype, void* out, int64_t ldo, void* workspace,
                        size_t workspace_bytes, spectra_stream_t stream);

@@ -58,6 +58,7 @@ SIGNATURES = {
     "spectra_w4a16_gemv_fused": (c_int32, [ctypes.POINTER(QWeight), c_void_p, c_int64, c_int32, c_int32,
                                            ctypes.POINTER(GemvFusion), c_void_p, c_int64, c_void_p]),
     "spectra_w4a16_gemm_workspace": (c_size_t, [ctypes.POINTER(QWeight), c_int64, c_int32]),
+    "spectra_w4a16_gemm_mid": (c_int32, [ctypes.POINTER(QWeight), c_int64, c_size_t]),
     "spectra_w4a16_gemm": (c_int32, [ctypes.POINTER(QWeight), c_void_p, c_int64, c_int64, c_int32,
                                      c_void_p, c_int64, c_void_p, c_size_t, c_void_p]),
     "spectra_w4a16_linear": (c_int32, [ctypes.POINTER(QWeight), c_void_p, c_int64, c_int64, c_int32,

@@ -606,6 +606,8 @@ size_t mid_workspace(const spectra_qweight_t* w, int64_t m, int64_t tile_wgs);
 int mid_launch(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m, int act_dtype, void* out,
                int64_t ldo, void* workspace, size_t workspace_bytes, int64_t tile_wgs, hipStream_t s);
 
+bool mid_runs(const spectra_qweight_t* w, int64_t m, size_t workspace_bytes, int64_t tile_wgs);
+
 // skinny.hip: the small-batch MFMA family (2 <= m <= 16)
 size_t skinny_workspace(const spectra_qweight_t* w, int64_t m);
 int skinny_launch(const spectra_qweight_t* w, const void* x, int64_t ldx, int64_t m, int act_dtype, void* out,
@@ -643,6 +645,10 @@ extern "C" size_t spectra_w4a16_gemm_workspace(const spectra_qweight_t* w, int64
   const size_t need = gemm_workspace_min(w, m), lib = prefill_workspace(w, m, act_dtype);
   const size_t mid = mid_workspace(w, m, tile_workgroups(w, m));
   return std::max(need, std::max(lib, mid));
+}
+
+extern "C" int spectra_w4a16_gemm_mid(const spectra_qweight_t* w, int64_t m, size_t workspace_bytes) {
+  return validate_qweight(w) == SPECTRA_OK && m > 0 && mid_runs(w, m, workspace_bytes, tile_workgroups(w, m));
 }
 
 extern "C" int spectra_w4a16_gemm(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m,

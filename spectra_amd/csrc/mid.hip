@@ -854,21 +854,34 @@ static int64_t mid_entries_count(const spectra_qweight_t* w) {
   return 0;
 }
 
-// When this family runs.  Whole calls, us, it against the 256-row-tile GEMM (four decoder layers,
-// N x K = 5120 x 3072, 3072 x 3072, 16384 x 3072, 3072 x 8192; NF4, 0.5% outliers): 48 rows 26.8 /
-// 24.9 / 41.4 / 32.6 against 30.2 / 26.9 / 49.1 / 43.3, 96 rows 31.7 / 28.1 / 53.2 / 37.6 against
-// 34.3 / 30.7 / 52.8 / 44.6, 160 rows 39 / 36 / 73 / 54 against 37 / 35 / 58 / 47: an outlier entry
-// costs a read of every row's activation here and a fixed amount there, so with outliers the line
-// lies at 96 rows.  Without: 200 rows 34 / 30 / 56 / 40 against 32 / 30 / 53 / 41, 160 rows 29 / 27 /
-// 45 / 35 against 32 / 30 / 51 / 41.  Where that GEMM leaves most of the chip idle (it splits K at
-// most eight ways, and not at all for N % 4 != 0) this family is faster at any size: N = 289,
-// K = 12288 31 against 259 at 130 rows, 43 against 279 at 400; N = 1001, K = 2112 36 against 67.
+// When this family runs.  Whole calls in graphs over 450 MB of layers, us, the 256-row-tile GEMM / this
+// family, N x K = 5120 x 3072, 16384 x 3072, 3072 x 8192, 14336 x 4096:
+//   NF4, none      32 rows  25 / 18   44 / 25   36 / 20   55 / 27    96 rows  30 / 26   50 / 36   41 / 27   61 / 38
+//   NF4, 0.5%      32 rows  27 / 24   46 / 35   39 / 28   58 / 38    48 rows  29 / 29   48 / 42   40 / 34   59 / 45
+//                  96 rows  33 / 34   53 / 56   42 / 38   64 / 59
+//   NF4, 2%        32 rows  32 / 28   51 / 45   49 / 38   65 / 51    48 rows  32 / 36   53 / 57   50 / 51   67 / 67
+//   Format A, 1%   32 rows  29 / 25   52 / 41   44 / 32   64 / 45    48 rows  31 / 30   54 / 48   45 / 40   65 / 55
+//                  96 rows  35 / 36   58 / 63   48 / 43   69 / 72
+// An outlier entry costs a read of every row's activation here and a fixed amount there, so the line is
+// a density that falls with the rows; it lies twice as high for K >= 4096 (that GEMM's chain of K steps
+// is what it is up against), and for Format A (its decode needs no table here) up to 64 rows or for
+// K >= 8192, and small weights with short rows lose to the reduce's fixed part (2048 x 2048, 0.5%, 56
+// rows 21.8 / 23.3).  Without outliers 160 rows are 33 / 30, 55 / 49, 42 / 36, 64 / 53, and 224 rows
+// slower here.  Where that GEMM leaves most of the chip idle (it splits K at most eight ways, and not
+// at all for N % 4 != 0) this family is faster at any size: N = 289, K = 12288 31
+// against 259 at 130 rows, 43 against 279 at 400; N = 1001, K = 2112 36 against 67.
 static bool mid_serves(const spectra_qweight_t* w, int64_t m, int64_t tile_wgs) {
+  const int64_t entries = mid_entries_count(w);
   if (m < 17 || m >= 512 || w->n < 1 || w->k < 64 || w->k % 64 != 0 || w->k > 32768 || w->hadamard_block > 512 ||
-      (w->format == SPECTRA_FMT_NF4 && w->group_size < 32) || mid_entries_count(w) >= (1LL << 31) ||
-      w->n > 65535 * 32)
+      (w->format == SPECTRA_FMT_NF4 && w->group_size < 32) || entries >= (1LL << 31) - 4096 || w->n > 65535 * 32)
     return false;
-  return m <= (mid_entries_count(w) > 0 ? 96 : 160) || tile_wgs < device_cu_count() / 4;
+  if (tile_wgs < device_cu_count() / 4) return true;
+  if (entries == 0) return m <= 160;
+  int64_t per = m <= 32 ? 40 : m <= 64 ? 160 : 320;  // weights to an entry, at least
+  if (m > 32 && w->k >= 4096) per /= 2;
+  if (m > 32 && (m <= 64 || w->k >= 8192) && w->format == SPECTRA_FMT_ASYM_G32) per /= 2;
+  const int64_t fixed = m > 32 && w->k < 4096 ? 1 << 22 : 0;
+  return m <= 96 && entries * per + fixed <= w->n * w->k;
 }
 
 struct MidWorkspace {
@@ -893,6 +906,10 @@ size_t mid_workspace(const spectra_qweight_t* w, int64_t m, int64_t tile_wgs) {
   return mid_serves(w, m, tile_wgs) ? mid_layout(w, m, plan_mid(m, w->n, w->k)).total : 0;
 }
 
+bool mid_runs(const spectra_qweight_t* w, int64_t m, size_t workspace_bytes, int64_t tile_wgs) {
+  return mid_serves(w, m, tile_wgs) && workspace_bytes >= mid_layout(w, m, plan_mid(m, w->n, w->k)).total;
+}
+
 template <int FMT>
 static const void* mid_pick(const MidPlan& g) {
   if (g.cs == 1) return g.t == 3 ? (const void*)mid_kernel<FMT, 3, 1> : (const void*)mid_kernel<FMT, 4, 1>;
@@ -903,10 +920,9 @@ static const void* mid_pick(const MidPlan& g) {
 // SPECTRA_ERR_UNSUPPORTED (nothing launched): the caller runs the 256-row-tile GEMM
 int mid_launch(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m, int act_dtype, void* out,
                int64_t ldo, void* workspace, size_t workspace_bytes, int64_t tile_wgs, hipStream_t s) {
-  if (!mid_serves(w, m, tile_wgs)) return SPECTRA_ERR_UNSUPPORTED;
+  if (!mid_runs(w, m, workspace_bytes, tile_wgs)) return SPECTRA_ERR_UNSUPPORTED;
   const MidPlan g = plan_mid(m, w->n, w->k);
   const MidWorkspace l = mid_layout(w, m, g);
-  if (workspace_bytes < l.total) return SPECTRA_ERR_UNSUPPORTED;
   const bool has_o = mid_entries_count(w) > 0, csr = w->outlier_kind == SPECTRA_OUTLIERS_CSR;
   uint8_t* ws = (uint8_t*)workspace;
   int gs = 0;

@@ -132,3 +132,36 @@ def test_decode_kernels_reject_bad_arguments():
     assert lib.spectra_silu_mul(p, 100, 1, 64, p, None) == L.ERR_INVALID
     assert lib.spectra_greedy_next(p, 0, p, None, 0, None, None) == L.ERR_INVALID
     assert lib.spectra_greedy_next(p, 10, p, p, 10, None, None) == L.ERR_INVALID  # history needs pos
+
+
+def test_mid_size_rows_by_outlier_density():
+    """Which calls of 17 .. 511 rows run on the mid-size family (256 CUs assumed without a device):
+    all up to 160 rows without outliers; with them a density that falls with the rows, is higher for
+    K >= 4096 and for Format A, and spares small weights; never without its workspace; any density
+    where the 256-row tiles would leave most of the chip idle."""
+    lib = L.load()
+
+    def mid(m, n, k, ratio, fmt=L.FMT_NF4, ws=1 << 40):
+        asym = fmt == L.FMT_ASYM_G32
+        w = _desc(n=n, k=k, format=fmt, group_size=32 if asym else 64, packed_stride=k // 2, scales_stride=k // 32)
+        if asym:
+            w.zeros, w.zeros_stride = 0x3000, k // 32
+        if ratio and asym:
+            w.outlier_kind, w.num_outliers = L.OUTLIERS_COLUMNS, int(k * ratio)
+            w.outlier_idx, w.outlier_w, w.outlier_w_stride = 0x4000, 0x5000, w.num_outliers
+        elif ratio:
+            w.outlier_kind, w.csr_nnz = L.OUTLIERS_CSR, int(n * k * ratio)
+            w.csr_rowptr, w.csr_col, w.csr_val = 0x4000, 0x5000, 0x6000
+        return lib.spectra_w4a16_gemm_mid(ctypes.byref(w), m, ws)
+
+    A = L.FMT_ASYM_G32
+    for shape in ((5120, 3072), (16384, 3072), (3072, 8192), (14336, 4096)):
+        assert [mid(m, *shape, 0.0) for m in (16, 17, 160, 161, 600)] == [0, 1, 1, 0, 0], shape
+        assert mid(32, *shape, 0.02) and not mid(32, *shape, 0.05) and not mid(97, *shape, 0.005), shape
+        assert not mid(32, *shape, 0.0, ws=1 << 20), shape
+    assert not mid(96, 16384, 3072, 0.005) and not mid(96, 16384, 3072, 0.01) and not mid(48, 16384, 3072, 0.01)
+    assert mid(48, 16384, 3072, 0.005) and mid(96, 16384, 3072, 0.0025)
+    assert mid(48, 3072, 8192, 0.01) and mid(96, 3072, 8192, 0.005) and not mid(96, 3072, 8192, 0.01)
+    assert mid(48, 16384, 3072, 0.01, A) and mid(96, 3072, 8192, 0.01, A) and not mid(96, 14336, 4096, 0.01, A)
+    assert not mid(48, 2048, 2048, 0.005) and mid(32, 2048, 2048, 0.005)
+    assert mid(400, 289, 12288, 0.02)
