@@ -36,6 +36,33 @@ def test_attend_long(hip, heads, kv, hd, L, positions):
         assert (out.double() - ref).abs().max().item() <= 2.0 ** -10 * vd.abs().max().item(), p
 
 
+@pytest.mark.parametrize("heads,kv,hd,L,positions", [
+    (6, 2, 128, 9000, (0, 130, 4096, 4223, 8192, 8999)), (8, 1, 64, 5000, (127, 4100, 4999)),
+    (4, 2, 256, 5000, (128, 4097, 4999))])
+def test_attend_long_rope(hip, heads, kv, hd, L, positions):
+    """With the rotation: the query heads and the new key, appended from a workgroup's first, second or
+    third span, as fp32 products and sums rounded to fp16 once (the key bit for bit).  Bound as above."""
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    k0, v0 = (torch.randn(kv, L, hd, generator=g, device="cuda").half() for _ in range(2))
+    ang = torch.rand(L, hd // 2, generator=g, device="cuda") * 6.3
+    cos, sin = ang.cos().contiguous(), ang.sin().contiguous()
+    ws = torch.zeros(K.attend_workspace_bytes(heads, hd, L), dtype=torch.uint8, device="cuda")
+    for p in positions:
+        k, v = k0.clone(), v0.clone()
+        k[:, p:], v[:, p:] = float("nan"), float("nan")
+        qkv = torch.randn((heads + 2 * kv) * hd, generator=g, device="cuda").half()
+        out = K.attend_decode(qkv, torch.tensor([p], device="cuda"), cos, sin, heads, kv, k, v, ws)
+        row = qkv.view(-1, hd)
+        a, b = row[:heads + kv, :hd // 2].float(), row[:heads + kv, hd // 2:].float()
+        rot = torch.cat([a * cos[p] - b * sin[p], b * cos[p] + a * sin[p]], 1).half()
+        assert torch.equal(k[:, p], rot[heads:]) and torch.equal(v[:, p], row[heads + kv:]), p
+        assert bool(k[:, p + 1:].isnan().all()) and torch.equal(k[:, :p], k0[:, :p])
+        kd, vd = (t[:, :p + 1].double().repeat_interleave(heads // kv, 0) for t in (k, v))
+        s = (kd * rot[:heads].double()[:, None]).sum(-1) / math.sqrt(hd)
+        ref = (torch.softmax(s, -1)[..., None] * vd).sum(1)
+        assert (out.double() - ref).abs().max().item() <= 2.0 ** -10 * vd.abs().max().item(), p
+
+
 @pytest.mark.parametrize("L,rows", [(2049, (0, 16)), (9000, (0, 16)), (9000, (4096, 4112)), (9000, (128, 9000))])
 def test_attend_long_infinite_scores(hip, L, rows):
     """Scores of -inf weigh nothing, also over all 16 rows that a wave takes of a span, in its first

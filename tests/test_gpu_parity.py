@@ -649,8 +649,9 @@ def test_dense_outlier_rows(hip):
 
 @pytest.mark.parametrize("m", [40, 300])
 def test_gemm_split_k_outliers_across_splits(hip, m):
-    """Few output tiles -> the GEMM splits K (8 splits of 512 here); outlier runs that cross
-    split boundaries, a fully dense row and a bias must land in exactly one split each."""
+    """Few output tiles -> K is split (on the mid-size family here; test_mid_gemm.py runs the
+    256-row tiles' 8 splits of 512); outlier runs that cross split boundaries, a fully dense row
+    and a bias must land in exactly one split each."""
     case(m=m)
     n, k = 256, 4096
     rng = np.random.default_rng(m)

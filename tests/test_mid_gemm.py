@@ -1,5 +1,6 @@
-"""The mid-size batch family (17 rows up to 96, 160 without outliers, 511 on shapes with few tiles)
-against the float64 product of W_eff, at the edges of its tiles: 32-row tiles and the change from
+"""The mid-size batch family (17 rows up to 96 by outlier density, 160 without outliers, 511 on shapes
+with few tiles) and the 256-row tiles beside it against the float64 product of W_eff, at the edges of
+the family's tiles: 32-row tiles and the change from
 four chunks a stage to two and to one, columns past the last 128, K of an odd number of 64-chunks and
 of a partial quad, every number of K splits' remainder, both formats and nibble orders, rotation
 blocks, dense and empty outlier rows, codes under the outliers that are not zero, unaligned and
@@ -37,6 +38,12 @@ def _dense(q, bs=64):
                          rp, q.col.cpu().numpy(), q.val.cpu().numpy(), blocksize=bs)
 
 
+def _runs_mid(hip, ops, m, dt):
+    """Whether a call with the workspace the library asks for runs on this family."""
+    adt = L.F16 if dt == "float16" else L.BF16
+    return bool(hip.spectra_w4a16_gemm_mid(ops.ptr(), m, hip.spectra_w4a16_gemm_workspace(ops.ptr(), m, adt)))
+
+
 def _check(y, x, w, had, bias, dt):
     xr = O.rotate_blocks(x.float().cpu().numpy(), had) if had else x.float().cpu().numpy()
     ref = torch.from_numpy(xr.astype(np.float64)).cuda() @ torch.from_numpy(w.astype(np.float64)).cuda().t()
@@ -46,21 +53,23 @@ def _check(y, x, w, had, bias, dt):
     assert rel <= (1e-3 if dt == "float16" else 5e-3), rel
 
 
-@pytest.mark.parametrize("m,n,k,had,ratio,marlin,dt,bs", [
-    (17, 128, 1024, 128, 0.01, True, "float16", 64),
-    (32, 129, 64, 64, 0.05, False, "bfloat16", 64),     # one chunk
-    (33, 1000, 1088, 64, 0.01, True, "float16", 32),    # 17 chunks, 32-blocks
-    (64, 3072, 3072, 512, 0.005, True, "float16", 64),
-    (65, 640, 2112, 32, 0.02, False, "float16", 64),    # 33 chunks
-    (96, 5120, 1024, 128, 0.005, True, "bfloat16", 64),
-    (97, 1537, 1024, 0, 0.0, True, "float16", 64),      # two chunks a stage, 4 row tiles
-    (129, 384, 1344, 0, 0.0, False, "float16", 64),     # one chunk a stage, 3 + 3 row tiles
-    (160, 2048, 2048, 256, 0.0, True, "bfloat16", 64),
-    (255, 129, 3072, 2, 0.01, True, "float16", 64),     # few tiles: any row count
-    (257, 77, 4096, 128, 0.01, False, "float16", 64),   # two row blocks
-    (511, 33, 6144, 0, 0.01, True, "float16", 128),
+@pytest.mark.parametrize("m,n,k,had,ratio,marlin,dt,bs,mid", [
+    (17, 128, 1024, 128, 0.01, True, "float16", 64, True),
+    (32, 129, 64, 64, 0.05, False, "bfloat16", 64, True),     # one chunk
+    (33, 1000, 1088, 64, 0.01, True, "float16", 32, True),    # 17 chunks, 32-blocks
+    (64, 3072, 3072, 512, 0.005, True, "float16", 64, False),  # (the 256-row tiles, by density)
+    (64, 3072, 3072, 512, 0.0025, True, "float16", 64, True),
+    (65, 640, 2112, 32, 0.02, False, "float16", 64, True),    # 33 chunks
+    (96, 5120, 1024, 128, 0.005, True, "bfloat16", 64, False),
+    (96, 5120, 2048, 128, 0.001, True, "bfloat16", 64, True),
+    (97, 1537, 1024, 0, 0.0, True, "float16", 64, True),      # two chunks a stage, 4 row tiles
+    (129, 384, 1344, 0, 0.0, False, "float16", 64, True),     # one chunk a stage, 3 + 3 row tiles
+    (160, 2048, 2048, 256, 0.0, True, "bfloat16", 64, True),
+    (255, 129, 3072, 2, 0.01, True, "float16", 64, True),     # few tiles: any row count
+    (257, 77, 4096, 128, 0.01, False, "float16", 64, True),   # two row blocks
+    (511, 33, 6144, 0, 0.01, True, "float16", 128, True),
 ])
-def test_mid_nf4(hip, m, n, k, had, ratio, marlin, dt, bs):
+def test_mid_nf4(hip, m, n, k, had, ratio, marlin, dt, bs, mid):
     q, _ = _nf4(n, k, had, ratio, marlin, bs)
     g = torch.Generator(device="cuda").manual_seed(m)
     x = torch.randn(m, k, generator=g, device="cuda").to(DT[dt])
@@ -68,17 +77,19 @@ def test_mid_nf4(hip, m, n, k, had, ratio, marlin, dt, bs):
     x[0] *= 1e-3
     bias = torch.randn(n, generator=g, device="cuda")
     col, val = q.outliers()
+    rowptr = q.rowptr if col is not None else None
+    ops = K.QWeightOperands(q.packed, q.absmax, None, k, codebook="nf4", group_size=bs, hadamard_block=had,
+                            marlin_layout=marlin, outlier_idx=col, outlier_w=val, outlier_rowptr=rowptr)
+    assert _runs_mid(hip, ops, m, dt) == mid
     y = K.batched_w4a16_gemm(x, q.packed, q.absmax, None, col, val, marlin, codebook="nf4", group_size=bs,
-                             hadamard_block=had, outlier_rowptr=q.rowptr if col is not None else None, bias=bias)
+                             hadamard_block=had, outlier_rowptr=rowptr, bias=bias)
     _check(y, x, _dense(q, bs), had, bias, dt)
 
 
-@pytest.mark.parametrize("m,n,k,n_out,marlin,dt", [
-    (17, 256, 96 * 2, 3, True, "float16"), (40, 1001, 2112, 20, False, "bfloat16"), (96, 3072, 3072, 30, True, "float16"),
-    (160, 640, 1024, 0, True, "float16"), (300, 99, 2048, 7, True, "float16")])
-def test_mid_format_a(hip, m, n, k, n_out, marlin, dt):
+def _format_a(m, n, k, n_out, marlin, dt):
+    """Operands, W_eff and activations; the codes under the outlier columns are not zero."""
     rng = np.random.default_rng(m + n)
-    qc = rng.integers(0, 16, (n, k)).astype(np.uint8)  # codes under the outlier columns are not zero
+    qc = rng.integers(0, 16, (n, k)).astype(np.uint8)
     z = rng.integers(0, 16, (n, k // 32)).astype(np.uint8)
     s = (rng.random((n, k // 32)) * 0.01 + 0.001).astype(np.float16)
     packed = O.pack_nibbles(qc, marlin)
@@ -90,9 +101,72 @@ def test_mid_format_a(hip, m, n, k, n_out, marlin, dt):
         w[:, idx] = ow.float().cpu().numpy()
     g = torch.Generator(device="cuda").manual_seed(m)
     x = torch.randn(m, k, generator=g, device="cuda").to(DT[dt])
-    y = K.batched_w4a16_gemm(x, torch.from_numpy(packed).cuda(), torch.from_numpy(s).cuda(), torch.from_numpy(z).cuda(),
-                             torch.from_numpy(idx).cuda() if n_out else None, ow, marlin)
-    _check(y, x, w, 0, None, dt)
+    args = (torch.from_numpy(packed).cuda(), torch.from_numpy(s).cuda(), torch.from_numpy(z).cuda(),
+            torch.from_numpy(idx).cuda() if n_out else None, ow, marlin)
+    ops = K.QWeightOperands(*args[:3], k, marlin_layout=marlin, outlier_idx=args[3], outlier_w=ow)
+    return args, ops, w, x
+
+
+@pytest.mark.parametrize("m,n,k,n_out,marlin,dt,mid", [
+    (17, 256, 96 * 2, 3, True, "float16", True), (40, 1001, 2112, 20, False, "bfloat16", True),
+    (96, 3072, 3072, 30, True, "float16", False), (96, 3072, 3072, 4, True, "float16", True),
+    (160, 640, 1024, 0, True, "float16", True), (300, 99, 2048, 7, True, "float16", True),
+    (128, 1536, 1024, 0, False, "float16", True),    # two chunks a stage, 4 row tiles
+    (255, 77, 1024, 3, True, "bfloat16", True),      # one chunk a stage, 4 + 4 row tiles
+    (511, 65, 1088, 5, False, "float16", True)])
+def test_mid_format_a(hip, m, n, k, n_out, marlin, dt, mid):
+    args, ops, w, x = _format_a(m, n, k, n_out, marlin, dt)
+    assert _runs_mid(hip, ops, m, dt) == mid
+    _check(K.batched_w4a16_gemm(x, *args), x, w, 0, None, dt)
+
+
+def _on_tiles(hip, ops, x, n):
+    """The product on the 256-row tiles: where the mid-size family serves the call, in the largest
+    workspace that does not hold its buffers."""
+    m, k = x.shape
+    adt = L.F16 if x.dtype == torch.float16 else L.BF16
+    size = hip.spectra_w4a16_gemm_workspace(ops.ptr(), m, adt)
+    if hip.spectra_w4a16_gemm_mid(ops.ptr(), m, size):
+        lo = 0
+        while size - lo > 1:
+            at = (lo + size) // 2
+            lo, size = (lo, at) if hip.spectra_w4a16_gemm_mid(ops.ptr(), m, at) else (at, size)
+        size = lo
+    ws = torch.empty(size, device="cuda", dtype=torch.uint8)
+    out = torch.empty(m, n, device="cuda", dtype=x.dtype)
+    L.check("spectra_w4a16_gemm", hip.spectra_w4a16_gemm(
+        ops.ptr(), x.data_ptr(), x.stride(0), m, adt, out.data_ptr(), n, ws.data_ptr(), size,
+        torch.cuda.current_stream().cuda_stream))
+    return out
+
+
+@pytest.mark.parametrize("m,n,k,had", [(40, 256, 4096, 128), (300, 256, 4096, 128), (33, 130, 1024, 0), (97, 512, 3072, 64)])
+def test_tiles_nf4_split_k_outliers(hip, m, n, k, had):
+    """The 256-row tiles on shapes that split K (8 splits of 512 at K = 4096): entries on both sides of
+    every split's edge, a fully dense row, a half-dense one and an empty one."""
+    g = torch.Generator(device="cuda").manual_seed(m)
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    mask = torch.rand(n, k, generator=g, device="cuda") < 0.005
+    mask[3, 480:560] = True
+    mask[n - 2, 1000:1100] = True
+    mask[77, :] = True
+    mask[n - 1, ::2] = True
+    mask[5] = False
+    q = C.quantize_nf4(torch.where(mask, w * 10, w).half(), 64, 0, mask, True)
+    ops = K.QWeightOperands(q.packed, q.absmax, None, k, codebook="nf4", hadamard_block=had, marlin_layout=True,
+                            outlier_idx=q.col, outlier_w=q.val, outlier_rowptr=q.rowptr)
+    x = torch.randn(m, k, generator=g, device="cuda").half()
+    y = _on_tiles(hip, ops, x, n)
+    _check(y, x, _dense(q), had, None, "float16")
+    assert torch.equal(_on_tiles(hip, ops, x, n), y)  # the split partials are summed in a fixed order
+
+
+@pytest.mark.parametrize("m,n,k,n_out,marlin,dt", [
+    (130, 8192, 1024, 10, True, "float16"), (300, 8192, 512, 3, False, "bfloat16"), (33, 256, 4096, 20, True, "float16"),
+    (40, 1000, 1024, 12, False, "float16")])
+def test_tiles_format_a(hip, m, n, k, n_out, marlin, dt):
+    args, ops, w, x = _format_a(m, n, k, n_out, marlin, dt)
+    _check(_on_tiles(hip, ops, x, n), x, w, 0, None, dt)
 
 
 def test_mid_strides_alignment_and_workspace(hip):
@@ -107,14 +181,13 @@ def test_mid_strides_alignment_and_workspace(hip):
     out = torch.full((m, n + 3), 7.0, device="cuda", dtype=torch.float16)
     need = hip.spectra_w4a16_gemm_workspace(ops.ptr(), m, L.F16)
     stream = torch.cuda.current_stream().cuda_stream
-    small = next(b for b in range(1 << 16, need, 4096) if b >= m * k * 2 + (1 << 17))
-    for off, size in ((1, need), (0, need), (0, min(small, need - 1))):
+    small = next(b for b in range(need, 0, -256) if not hip.spectra_w4a16_gemm_mid(ops.ptr(), m, b))
+    assert small < need
+    for off, size in ((1, need), (0, need), (0, small)):
         x = xb[:, off:off + k]
         ws = torch.empty(size, device="cuda", dtype=torch.uint8)
         st = hip.spectra_w4a16_gemm(ops.ptr(), x.data_ptr(), xb.stride(0), m, L.F16, out.data_ptr(), out.stride(0),
                                     ws.data_ptr(), size, stream)
-        if st == L.ERR_WORKSPACE and size < need:
-            continue  # (also smaller than that GEMM needs: refused, nothing launched)
         assert st == 0
         _check(out[:, :n], x, _dense(q), 128, None, "float16")
         assert bool((out[:, n:] == 7.0).all())
