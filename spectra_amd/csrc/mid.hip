@@ -920,9 +920,10 @@ static const void* mid_pick(const MidPlan& g) {
 // SPECTRA_ERR_UNSUPPORTED (nothing launched): the caller runs the 256-row-tile GEMM
 int mid_launch(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m, int act_dtype, void* out,
                int64_t ldo, void* workspace, size_t workspace_bytes, int64_t tile_wgs, hipStream_t s) {
-  if (!mid_runs(w, m, workspace_bytes, tile_wgs)) return SPECTRA_ERR_UNSUPPORTED;
+  if (!mid_serves(w, m, tile_wgs)) return SPECTRA_ERR_UNSUPPORTED;
   const MidPlan g = plan_mid(m, w->n, w->k);
   const MidWorkspace l = mid_layout(w, m, g);
+  if (workspace_bytes < l.total) return SPECTRA_ERR_UNSUPPORTED;  // (as mid_runs)
   const bool has_o = mid_entries_count(w) > 0, csr = w->outlier_kind == SPECTRA_OUTLIERS_CSR;
   uint8_t* ws = (uint8_t*)workspace;
   int gs = 0;
