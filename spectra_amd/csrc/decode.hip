@@ -317,13 +317,14 @@ __device__ __forceinline__ float load_dev(const float* p) {
 // partial stores have completed before the workgroup counts itself in (one device-scope
 // atomic on the head's counter, 256 bytes apart per head); the workgroup that brings the
 // count to nspan merges the G (<= 8) heads' spans exactly as a separate merge kernel would
-// and leaves the counter at 0.  Spans are merged in batches of 16 (one batch up to 1024
-// positions), every load of a batch in flight at once: lane (j, u) of the first 16 G
-// threads (16-lane rows: j = tid / 16, u = tid % 16) loads (m, l) of head j, span u of the
-// batch and, with 16-lane reductions, keeps the head's running maximum and sum of
-// exponentials and turns the batch into weights exp(m - M) (m = -inf marks an empty span,
-// weight 0) in LDS; every thread loads the V sums of its outputs (o, o + 256, ...) and folds
-// them in with those weights.
+// and leaves the counter at 0.  A workgroup's piece is one span, or on long caches several.  Pieces
+// are merged in batches of B (16: one batch up to 1024 positions; 32 for the 8-wave workgroups, whose
+// heads have at most 32), every load of a batch in flight at once: lane (j, u) of the first B G
+// threads (B-lane rows: j = tid / B, u = tid % B) loads (m, l) of head j, piece u of the
+// batch and, with B-lane reductions, keeps the head's running maximum and sum of
+// exponentials and turns the batch into weights exp(m - M) (m = -inf marks an empty piece,
+// weight 0) in LDS; every one of the NT threads loads the V sums of its outputs (o, o + NT, ...) and
+// folds them in with those weights.
 template <int HD, int NT = kDecThreads, int B = 16>
 __device__ __forceinline__ void attend_arrive_merge(const float* part, uint32_t* counter, uint16_t* out, int kh,
                                                     int G, int nspan, int tid, int* last_l) {
@@ -1228,7 +1229,9 @@ static int attend_launch(const void* qkv, const int64_t* pos, const float* cos_t
   // after: 24 / 8 heads, position 6001 of 8192, 20.9 and 13.0 (24.6 MB: 5.1 at the card's copy
   // rate, on the 7.6 of a 700-position call); position 300 of 16384, 37.9 and 10.4; 32 / 4 heads,
   // 15000 of 16384, 46.9 and 18.5.  16 waves took 14.1 / 14.6 / 18.3, 64 pieces 14.7 / 15.3 / 18.2,
-  // several spans on 4 waves 15.6 / 9.8 / 28.1; 1900 of 2048 takes 9.1 as it was.
+  // several spans on 4 waves 15.6 / 9.8 / 28.1; 1900 of 2048 takes 9.1 as it was.  One KV head (8
+  // query heads), which this leaves at 32 workgroups: 8183 of 8192 24.7 and 13.3, 16375 of 16384 42.9
+  // and 16.5, 65527 of 65536 152 and 37.5 (64 pieces 26.9, but 12.3 against 9.9 at 300 of 16384).
   int nspan = spectra_attend_spans(kvc.lmax);
   const bool wide = mfma && nspan > kAttendGrid;
   const int nw = wide ? 8 : 4;

@@ -70,8 +70,8 @@ __device__ __forceinline__ uint32_t f2bf_pair(float lo, float hi) {
 // nibble orders the 16 bytes of run c hold elements 32 c .. 32 c + 31 under one scale (group
 // size a multiple of 32): with the marlin pairs (k, k + 16) a lane reads kE bytes and takes
 // their low (first half of the run) or high nibbles, in the natural order kE / 2 bytes and
-// both nibbles.  All of a segment's loads (packed bytes, scales, outlier
-// entries) are issued before the first decode.  The NF4 codes come from a 16-entry LDS table.  Same
+// both nibbles.  All of a segment's loads (packed bytes, outlier entries, for 16-bit outputs the scales
+// too: kScalesAhead) are issued before the first decode.  The NF4 codes come from a 16-entry LDS table.  Same
 // values and roundings as dequant_kernel.  A pass's outliers are written over its rounded values in
 // the wave's 1 KB LDS slot, which all 64 lanes do (a partial pass too: an idle lane may hold an
 // entry), and the whole lines then go out once; only entries past the kDqPre * 64 that the wave holds

@@ -681,7 +681,8 @@ extern "C" int spectra_w4a16_gemm(const spectra_qweight_t* w, const void* a, int
     const int pst = prefill_launch(w, a, lda, m, act_dtype, out, ldo, workspace, workspace_bytes, s);
     if (pst != SPECTRA_ERR_UNSUPPORTED) return pst;
   }
-  // 17 .. 96 rows, to 160 without outliers, and shapes that leave this file's tiles few workgroups
+  // 17 .. 96 rows by outlier density, to 160 without outliers, and shapes that leave this file's tiles
+  // few workgroups
   const int mst = mid_launch(w, a, lda, m, act_dtype, out, ldo, workspace, workspace_bytes, tile_workgroups(w, m), s);
   if (mst != SPECTRA_ERR_UNSUPPORTED) return mst;
   uint16_t* a16 = (uint16_t*)workspace;
