@@ -648,7 +648,8 @@ extern "C" size_t spectra_w4a16_gemm_workspace(const spectra_qweight_t* w, int64
 }
 
 extern "C" int spectra_w4a16_gemm_mid(const spectra_qweight_t* w, int64_t m, size_t workspace_bytes) {
-  return validate_qweight(w) == SPECTRA_OK && m > 0 && mid_runs(w, m, workspace_bytes, tile_workgroups(w, m));
+  return validate_qweight(w) == SPECTRA_OK && m > 0 && workspace_bytes >= gemm_workspace_min(w, m) &&
+         mid_runs(w, m, workspace_bytes, tile_workgroups(w, m));
 }
 
 extern "C" int spectra_w4a16_gemm(const spectra_qweight_t* w, const void* a, int64_t lda, int64_t m,
